@@ -1211,7 +1211,23 @@ static int upload(Batch& b) {
   F2D_HIP(hipMemcpyAsync(v.islandData, islandData.data(), sizeof(int) * islandData.size(), hipMemcpyHostToDevice, b.stream));
   F2D_HIP(hipMemcpyAsync(v.contactLinks, links.data(), sizeof(int4) * totalContacts, hipMemcpyHostToDevice, b.stream));
   F2D_HIP(hipStreamSynchronize(b.stream));
-  for (SizeClass& c : b.classes) c.launch.continuous = b.launch.continuous;
+  for (SizeClass& c : b.classes) {
+    c.launch.continuous = b.launch.continuous;
+    c.launch.bulletLds = 0;
+  }
+  // LDS for the proxies that bullets sweep against (20 B per shape), only where some
+  // world of a class has bullets: it costs the other classes workgroups per compute unit
+  int bulletShapes = 0;
+  for (size_t i = 0; i < b.worlds.size(); ++i) {
+    const HostWorld& hw = b.worlds[i];
+    const bool bullets = std::any_of(hw.sims.begin(), hw.sims.end(), [](const BodySim& s) { return s.flags & BF_BULLET; });
+    const int bytes = 20 * (int)hw.shapes.size();
+    if (!bullets || bytes > 40960) continue;
+    bulletShapes = std::max(bulletShapes, bytes);
+    int& lds = b.classes[b.classOf[i]].launch.bulletLds;
+    lds = std::max(lds, bytes);
+  }
+  b.launch.bulletLds = bulletShapes;
   b.hostDirty = false;
   return 0;
 }

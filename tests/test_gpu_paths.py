@@ -1,0 +1,73 @@
+"""The device's launch paths against the C oracle at the sizes where a path begins or ends.
+
+A world is a container of bodies whose shapes are a fixture's, so that their geometry
+records are the reference's own; every step is compared as tests/test_gpu_oracle.py
+compares it, bit for bit, with the oracle stepping the device's previous state.
+"""
+import os
+
+import numpy as np
+import pytest
+
+import forge2d_amd as F
+from forge2d_amd import scenes
+from forge2d_amd import snapshot as S
+from oracle import pyoracle as O
+from tests.conftest import GOLDEN, load_fixture
+from tests.test_gpu_oracle import compare
+
+pytestmark = pytest.mark.gpu
+GEOM_BYTES = 148
+
+
+def container(bodies: int, seed: int, bullets: float = 0.0, sleep: bool = False, speed: float = 0.0,
+              columns: int = 0) -> tuple[bytes, bytes]:
+    """(spec, geometry records) of a world of `bodies` dynamic bodies in rows in a
+    container, their shapes drawn from the "mixed" fixture's dynamic ones."""
+    src, _, _ = load_fixture("mixed")
+    (_, fb, fs, _), = scenes.parse(src)
+    fg = np.load(os.path.join(GOLDEN, "mixed.npz"))["geoms"].reshape(-1, GEOM_BYTES)
+    dynamic = np.flatnonzero((fb["type"][fs["body"]] == scenes.DYNAMIC) & (fs["kind"] != scenes.K_SEGMENT))
+    walls = np.flatnonzero(fs["kind"] == scenes.K_SEGMENT)
+    hw = np.abs(fs["data"][walls][:, [0, 2]]).max()
+    rng = np.random.default_rng(seed)
+    pick = rng.choice(dynamic, bodies)
+    columns = columns or int((2.0 * hw - 2.0) / 1.7)
+    at = np.arange(bodies)
+    b = np.zeros(bodies + 1, scenes.BODY_DT)
+    b["qc"], b["gravity_scale"], b["sleep_threshold"] = 1.0, 1.0, 0.05
+    b["flags"] = scenes.BF_ENABLE_SLEEP | scenes.BF_AWAKE
+    b["type"][1:] = scenes.DYNAMIC
+    b["px"][1:] = 1.7 * (at % columns - (columns - 1) / 2.0) + rng.uniform(-0.1, 0.1, bodies)
+    b["py"][1:] = 1.0 + 1.3 * (at // columns) + rng.uniform(-0.1, 0.1, bodies)
+    b["vx"][1:], b["vy"][1:] = speed * rng.uniform(-1, 1, bodies), -speed * rng.random(bodies)
+    b["flags"][1:] |= np.where(rng.random(bodies) < bullets, scenes.BF_BULLET, 0).astype(np.int32)
+    s = np.concatenate([fs[walls], fs[pick]])
+    s["body"][:len(walls)], s["body"][len(walls):] = 0, 1 + at
+    h = scenes.world_header(sleep=sleep)
+    h["body_count"], h["shape_count"] = len(b), len(s)
+    spec = scenes.MAGIC + np.array([1, 0], "<i4").tobytes() + h.tobytes() + b.tobytes() + s.tobytes()
+    return spec, np.concatenate([fg[walls], fg[pick]]).tobytes()
+
+
+def follow(spec: bytes, geoms: bytes, steps: int, **batch):
+    b = F.Batch(spec, **batch)
+    raw = b.export(0)
+    prev = S.parse_one(raw)
+    for k in range(1, steps + 1):
+        b.step(steps=1)
+        assert b.sync() == 0
+        mine_raw = b.export(0)
+        mine = S.parse_one(mine_raw)
+        compare(mine, S.parse_one(O.step(spec, geoms, raw, prev).export()))
+        raw, prev = mine_raw, mine
+
+
+# bullets sweep against the proxies in query order from LDS up to 2,048 shapes a world and
+# from HBM above: one bullet, a few, more than a workgroup's 64 lanes, and either side of
+# the limit (the fixture's container has four walls)
+@pytest.mark.parametrize("bodies,bullets,sleep,steps", [(9, 1.0, False, 40), (70, 0.1, True, 40), (200, 0.6, False, 40),
+                                                        (2044, 0.05, False, 6), (2045, 0.05, False, 6)])
+def test_bullets(gpu, bodies, bullets, sleep, steps):
+    spec, geoms = container(bodies, 11 + bodies, bullets=bullets, sleep=sleep, speed=25.0)
+    follow(spec, geoms, steps)
