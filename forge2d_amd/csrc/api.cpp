@@ -853,17 +853,21 @@ static int deviceLdsLimit() {
 }
 
 // Lay out all worlds in flat arrays and allocate the device batch.
-// Dynamic LDS of a solve launch: the body states and per-step body terms (64 B per
-// body) of the class's largest world, its joints, plus room for `lanesPerBody`
-// constraint lanes per body (164 B each); a world whose joints or constraints do
-// not fit keeps them in HBM.
+// Dynamic LDS of a solve launch, for the class's largest world. Up to 1,024 bodies: the
+// body states and per-step body terms (64 B a body and one slot for the static bodies)
+// and the joints with their colour lists, which lets a world's contacts stay in the
+// workgroup's registers (solveResident). Larger worlds have more contacts than that and
+// keep only the body states (32 B a body) in LDS, up to the limit. lanesPerBody: room
+// beyond that, which no stage uses (0; the autotuner's trial sizes).
 static int solveLdsBytes(int maxBodies, int maxJoints, float lanesPerBody, int limit) {
-  const int bodies = std::max(maxBodies, 1) * (int)(sizeof(BodyState) + sizeof(BodyConst));
-  if (bodies > limit) return 0;
-  long total = bodies + (long)maxJoints * (long)sizeof(Joint) +
-               (long)(lanesPerBody * (float)std::max(maxBodies, 1)) * 4L * CN_FIELD_COUNT;
-  total = std::min<long>(total, limit);
-  return (int)((total + 255) & ~255L) <= limit ? (int)((total + 255) & ~255L) : limit;
+  const long bodies = std::max(maxBodies, 1);
+  const long states = bodies * (long)sizeof(BodyState);
+  long total = (bodies + 1) * (long)(sizeof(BodyState) + sizeof(BodyConst)) +
+               (long)maxJoints * (long)(sizeof(Joint) + sizeof(int));
+  if (bodies > 1024 || total > limit) total = states;
+  if (total > limit) return 0;
+  total += (long)(lanesPerBody * (float)bodies) * 4L * CN_FIELD_COUNT;
+  return (int)std::min<long>((total + 255) & ~255L, limit);
 }
 
 // LDS for the tree kernel's work arrays of a world's larger moving tree (worlds that
@@ -1009,8 +1013,9 @@ static int commit(Batch& b) {
     maxProxies = std::max(maxProxies, std::max(hw.tree[kDynamic].proxyCount, hw.tree[kKinematic].proxyCount));
   }
   b.launch.treeBlock = treeBlockFor(maxProxies);
-  int solve = maxBodies * (int)(sizeof(BodyState) + sizeof(BodyConst));
-  b.launch.solveLds = solve <= kLdsLimit ? ((solve + 255) & ~255) : 0;
+  int maxJoints = 0;
+  for (const HostWorld& hw : b.worlds) maxJoints = std::max(maxJoints, (int)hw.joints.size());
+  b.launch.solveLds = solveLdsBytes(maxBodies, maxJoints, 0.0f, deviceLdsLimit());
   if (b.launch.block == 0) b.launch.block = maxShapes <= 640 ? 64 : 256;
   // Full-batch launches dispatch the largest worlds first (longest-processing-time
   // order), so the last wave of workgroups holds the smallest worlds and the
@@ -1062,7 +1067,7 @@ static int commit(Batch& b) {
       c.launch.continuousChunks = c.maxBodies > 1024 ? (c.maxBodies + 63) / 64 : 0;
       // worlds of many thousand bodies run their solve stages over many workgroups
       c.launch.wideChunks = c.maxBodies > 4096 ? (c.maxBodies + 255) / 256 : 0;
-      c.launch.solveLds = solveLdsBytes(c.maxBodies, c.maxJoints, 1.0f, kLdsLimit);
+      c.launch.solveLds = solveLdsBytes(c.maxBodies, c.maxJoints, 0.0f, deviceLdsLimit());
       c.launch.treeLds = 0;
       int maxProxies = 0;
       for (int i : members[k]) {
@@ -1071,8 +1076,9 @@ static int commit(Batch& b) {
                                                    b.worlds[i].tree[kKinematic].proxyCount));
       }
       c.launch.treeBlock = treeBlockFor(maxProxies);
-      // one workgroup holds a whole world: the largest worlds get the most lanes
-      c.launch.block = c.limit <= 128 ? 64 : (c.limit <= 512 ? 128 : (c.limit <= 1024 ? 256 : 1024));
+      // a lane per body: the solve keeps kResidentLanes contacts a lane in registers, and
+      // the narrow phase takes a contact per lane and pass
+      c.launch.block = std::min(c.limit, 1024);
       if (b.forcedBlock) c.launch.block = b.forcedBlock;
       F2D_HIP(hipMalloc(&c.dList, sizeof(int) * c.count));
       F2D_HIP(hipMemcpy(c.dList, members[k].data(), sizeof(int) * c.count, hipMemcpyHostToDevice));
@@ -2130,10 +2136,10 @@ long f2dg_device_bytes(void* h) {
 
 // Step every world of the batch `steps` times: one launch per step, one workgroup per world.
 // Lane candidates of a size class for online tuning: 64, 128 and 256 lanes per
-// world, 256, 512 and 1024 for worlds of more than 512 shapes or bodies.
+// world, 128, 256 and 512 for worlds of more than 128 shapes or bodies, 256, 512 and
+// 1024 for worlds of more than 512.
 static int laneCandidate(const SizeClass& c, int k) {
-  static const int small[3] = {64, 128, 256}, large[3] = {256, 512, 1024};
-  return c.limit > 512 ? large[k] : small[k];
+  return (c.limit > 512 ? 256 : c.limit > 128 ? 128 : 64) << k;
 }
 
 // One online tuning round: three steps, step k with every class at its k-th lane
@@ -2689,7 +2695,7 @@ int f2dg_autotune(void* h, float dt, int subSteps, int steps, float* msOut) {
     int bestLds = c.launch.solveLds;
     for (int k = 0; k < 4; ++k) {
       LaunchConfig cfg = c.launch;
-      cfg.solveLds = solveLdsBytes(c.maxBodies, c.maxJoints, lanesPerBody[k], 65536);
+      cfg.solveLds = solveLdsBytes(c.maxBodies, c.maxJoints, lanesPerBody[k], deviceLdsLimit());
       F2D_HIP(hipEventRecord(e0, b->stream));
       for (int s = 0; s < steps; ++s) {
         if (f2d_launch_step(&b->dev.view, &sp, c.dList, c.count, b->stream, &cfg) != 0) return -1;

@@ -364,15 +364,20 @@ struct LaunchConfig {
                              // 256-lane workgroups
 };
 
-// Contact constraint lanes (one constraint per lane), S/contact_solver.c:1034-1064.
+// Contact constraint lanes (one constraint per lane), S/contact_solver.c:1034-1064, in
+// groups of four floats: a lane reads or writes a group with one 16-byte access, and the
+// lanes of a wavefront touch 1 KiB in a row.
 enum ConstraintField : int {
-  CN_INDEX_A = 0, CN_INDEX_B, CN_SLOT,
-  CN_INV_MASS_A, CN_INV_MASS_B, CN_INV_I_A, CN_INV_I_B,
-  CN_NX, CN_NY, CN_FRICTION, CN_TANGENT_SPEED, CN_ROLLING_RES, CN_ROLLING_MASS, CN_ROLLING_IMPULSE,
-  CN_BIAS_RATE, CN_MASS_SCALE, CN_IMPULSE_SCALE,
-  CN_A1X, CN_A1Y, CN_B1X, CN_B1Y, CN_BASE_SEP1, CN_NI1, CN_TNI1, CN_TI1, CN_NM1, CN_TM1,
-  CN_A2X, CN_A2Y, CN_B2X, CN_B2Y, CN_BASE_SEP2, CN_NI2, CN_TNI2, CN_TI2, CN_NM2, CN_TM2,
-  CN_RESTITUTION, CN_REL_VEL1, CN_REL_VEL2, CN_POINT_COUNT,
+  CN_INDEX_A = 0, CN_INDEX_B, CN_SLOT, CN_POINT_COUNT,
+  CN_NX, CN_NY, CN_FRICTION, CN_TANGENT_SPEED,
+  CN_A1X, CN_A1Y, CN_B1X, CN_B1Y,
+  CN_A2X, CN_A2Y, CN_B2X, CN_B2Y,
+  CN_BASE_SEP1, CN_BASE_SEP2, CN_NM1, CN_NM2,
+  CN_TM1, CN_TM2, CN_ROLLING_RES, CN_ROLLING_MASS,
+  CN_NI1, CN_TI1, CN_NI2, CN_TI2,
+  CN_TNI1, CN_TNI2, CN_ROLLING_IMPULSE, CN_PAD7,
+  CN_INV_MASS_A, CN_INV_I_A, CN_INV_MASS_B, CN_INV_I_B,
+  CN_RESTITUTION, CN_REL_VEL1, CN_REL_VEL2, CN_PAD9,
   CN_FIELD_COUNT
 };
 
@@ -391,7 +396,7 @@ struct BatchView {
   uint32_t* colorBits;
   int* overflow;        // overflow-colour contact ids in array order
   int* colorLists;      // per world at colorListOffset: colour arrays of colours 0..10
-  float* cons;          // constraint SoA: field f of lane i at cons[f * consStride + i]
+  float* cons;          // constraint lanes: group g (four fields) of lane i at cons[4 * (g * consStride + i)]
   long consStride;
   int* scratch;         // large-world sort scratch
   float4* sapBoxes;     // large-world sorted fat AABBs

@@ -32,9 +32,10 @@ inline int asInt(float v) {
 struct Cons {
   float* f;
   long stride;
-  F2D_HD float& operator()(int field, long lane) const { return f[field * stride + lane]; }
-  F2D_HD int geti(int field, long lane) const { return asInt(f[field * stride + lane]); }
-  F2D_HD void seti(int field, long lane, int v) const { f[field * stride + lane] = asFloat(v); }
+  F2D_HD float4& group(int g, long lane) const { return reinterpret_cast<float4*>(f)[g * stride + lane]; }
+  F2D_HD float& at(int field, long lane) const { return f[4 * ((field >> 2) * stride + lane) + (field & 3)]; }
+  F2D_HD int geti(int field, long lane) const { return asInt(at(field, lane)); }
+  F2D_HD void seti(int field, long lane, int v) const { at(field, lane) = asFloat(v); }
 };
 
 F2D_HD BodyState identityState() {
@@ -47,159 +48,113 @@ F2D_HD BodyState identityState() {
   return s;
 }
 
+#if defined(__HIP_DEVICE_COMPILE__)
+#define F2D_UNROLL2 _Pragma("unroll")
+#else
+#define F2D_UNROLL2
+#endif
+
+// One contact constraint's terms of the substeps, in registers.
+struct ContactLane {
+  float nx, ny, friction, tangentSpeed, rollingRes, rollingMass, rollingImpulse;
+  float ax[2], ay[2], bx[2], by[2];  // anchors
+  float sep[2], nm[2], tm[2];        // base separation, normal and tangent mass
+  float ni[2], ti[2], tni[2];        // normal, tangent and total normal impulses
+};
+// The inverse masses and inertias of its bodies (zero for a static body)
+struct ContactMass {
+  float mA, iA, mB, iB;
+};
+
 // ---------------------------------------------------------------------------- prepare
 
 // b2PrepareContactsTask lane body, S/contact_solver.c:1462-1627 (identical to the
-// overflow prepare :50-157 for the quantities both compute).
-F2D_HD void prepareContactLane(const Cons& c, long lane, const Contact& cs, int slot, int indexA, int indexB,
-                               float mA, float iA, float mB, float iB, const BodyState* states,
-                               Softness contactSoftness, Softness staticSoftness, float warmStartScale) {
+// overflow prepare :50-157 for the quantities both compute). relVel: the points'
+// relative normal velocities.
+F2D_HD void prepareLane(ContactLane& c, const Contact& cs, const ContactMass& k, const BodyState& sA,
+                        const BodyState& sB, float warmStartScale, float* relVel) {
   const Manifold& m = cs.m;
-  c.seti(CN_INDEX_A, lane, indexA);
-  c.seti(CN_INDEX_B, lane, indexB);
-  c.seti(CN_SLOT, lane, slot);
-  c.seti(CN_POINT_COUNT, lane, m.pointCount);
-  Vec2 vA = {0.0f, 0.0f};
-  float wA = 0.0f;
-  if (indexA >= 0) {
-    vA = states[indexA].v;
-    wA = states[indexA].w;
-  }
-  Vec2 vB = {0.0f, 0.0f};
-  float wB = 0.0f;
-  if (indexB >= 0) {
-    vB = states[indexB].v;
-    wB = states[indexB].w;
-  }
-  c(CN_INV_MASS_A, lane) = mA;
-  c(CN_INV_MASS_B, lane) = mB;
-  c(CN_INV_I_A, lane) = iA;
-  c(CN_INV_I_B, lane) = iB;
+  const float mA = k.mA, iA = k.iA, mB = k.mB, iB = k.iB;
   {
-    float k = iA + iB;
-    c(CN_ROLLING_MASS, lane) = k > 0.0f ? 1.0f / k : 0.0f;
+    float i = iA + iB;
+    c.rollingMass = i > 0.0f ? 1.0f / i : 0.0f;
   }
-  Softness soft = (indexA < 0 || indexB < 0) ? staticSoftness : contactSoftness;
   Vec2 normal = m.normal;
-  c(CN_NX, lane) = normal.x;
-  c(CN_NY, lane) = normal.y;
-  c(CN_FRICTION, lane) = cs.friction;
-  c(CN_TANGENT_SPEED, lane) = cs.tangentSpeed;
-  c(CN_RESTITUTION, lane) = cs.restitution;
-  c(CN_ROLLING_RES, lane) = cs.rollingResistance;
-  c(CN_ROLLING_IMPULSE, lane) = warmStartScale * m.rollingImpulse;
-  c(CN_BIAS_RATE, lane) = soft.biasRate;
-  c(CN_MASS_SCALE, lane) = soft.massScale;
-  c(CN_IMPULSE_SCALE, lane) = soft.impulseScale;
+  c.nx = normal.x;
+  c.ny = normal.y;
+  c.friction = cs.friction;
+  c.tangentSpeed = cs.tangentSpeed;
+  c.rollingRes = cs.rollingResistance;
+  c.rollingImpulse = warmStartScale * m.rollingImpulse;
   Vec2 tangent = rightPerp(normal);
+  const int pointCount = m.pointCount;
+  F2D_UNROLL2
   for (int p = 0; p < 2; ++p) {
-    const int o = p == 0 ? 0 : (CN_A2X - CN_A1X);
-    const int rvf = p == 0 ? CN_REL_VEL1 : CN_REL_VEL2;
-    if (p < m.pointCount) {
+    if (p < pointCount) {
       const ManifoldPoint& mp = m.points[p];
       Vec2 rA = mp.anchorA;
       Vec2 rB = mp.anchorB;
-      c(CN_A1X + o, lane) = rA.x;
-      c(CN_A1Y + o, lane) = rA.y;
-      c(CN_B1X + o, lane) = rB.x;
-      c(CN_B1Y + o, lane) = rB.y;
-      c(CN_BASE_SEP1 + o, lane) = mp.separation - dot(sub(rB, rA), normal);
-      c(CN_NI1 + o, lane) = warmStartScale * mp.normalImpulse;
-      c(CN_TI1 + o, lane) = warmStartScale * mp.tangentImpulse;
-      c(CN_TNI1 + o, lane) = 0.0f;
+      c.ax[p] = rA.x;
+      c.ay[p] = rA.y;
+      c.bx[p] = rB.x;
+      c.by[p] = rB.y;
+      c.sep[p] = mp.separation - dot(sub(rB, rA), normal);
+      c.ni[p] = warmStartScale * mp.normalImpulse;
+      c.ti[p] = warmStartScale * mp.tangentImpulse;
       float rnA = cross(rA, normal);
       float rnB = cross(rB, normal);
       float kNormal = mA + mB + iA * rnA * rnA + iB * rnB * rnB;
-      c(CN_NM1 + o, lane) = kNormal > 0.0f ? 1.0f / kNormal : 0.0f;
+      c.nm[p] = kNormal > 0.0f ? 1.0f / kNormal : 0.0f;
       float rtA = cross(rA, tangent);
       float rtB = cross(rB, tangent);
       float kTangent = mA + mB + iA * rtA * rtA + iB * rtB * rtB;
-      c(CN_TM1 + o, lane) = kTangent > 0.0f ? 1.0f / kTangent : 0.0f;
-      Vec2 vrA = add(vA, crossSV(wA, rA));
-      Vec2 vrB = add(vB, crossSV(wB, rB));
-      c(rvf, lane) = dot(normal, sub(vrB, vrA));
+      c.tm[p] = kTangent > 0.0f ? 1.0f / kTangent : 0.0f;
+      Vec2 vrA = add(sA.v, crossSV(sA.w, rA));
+      Vec2 vrB = add(sB.v, crossSV(sB.w, rB));
+      relVel[p] = dot(normal, sub(vrB, vrA));
     } else {
-      c(CN_A1X + o, lane) = 0.0f;
-      c(CN_A1Y + o, lane) = 0.0f;
-      c(CN_B1X + o, lane) = 0.0f;
-      c(CN_B1Y + o, lane) = 0.0f;
-      c(CN_BASE_SEP1 + o, lane) = 0.0f;
-      c(CN_NI1 + o, lane) = 0.0f;
-      c(CN_TI1 + o, lane) = 0.0f;
-      c(CN_TNI1 + o, lane) = 0.0f;
-      c(CN_NM1 + o, lane) = 0.0f;
-      c(CN_TM1 + o, lane) = 0.0f;
-      c(rvf, lane) = 0.0f;
+      c.ax[p] = c.ay[p] = c.bx[p] = c.by[p] = 0.0f;
+      c.sep[p] = c.nm[p] = c.tm[p] = c.ni[p] = c.ti[p] = 0.0f;
+      relVel[p] = 0.0f;
     }
+    c.tni[p] = 0.0f;
   }
 }
 
 // ---------------------------------------------------------------------------- coloured (SIMD lane order)
 
-F2D_HD BodyState gather(const BodyState* states, int idx) { return idx >= 0 ? states[idx] : identityState(); }
-F2D_HD void scatterVel(BodyState* states, int idx, const BodyState& b) {
-  if (idx >= 0) {
-    states[idx].v = b.v;
-    states[idx].w = b.w;
-  }
-}
-
 // b2WarmStartContactsTask lane, S/contact_solver.c:1671-1727
-F2D_HD void warmStartLane(const Cons& c, long lane, BodyState* states) {
-  int ia = c.geti(CN_INDEX_A, lane), ib = c.geti(CN_INDEX_B, lane);
-  BodyState bA = gather(states, ia);
-  BodyState bB = gather(states, ib);
-  float mA = c(CN_INV_MASS_A, lane), mB = c(CN_INV_MASS_B, lane);
-  float iA = c(CN_INV_I_A, lane), iB = c(CN_INV_I_B, lane);
-  float nx = c(CN_NX, lane), ny = c(CN_NY, lane);
-  float tx = ny;
-  float ty = 0.0f - nx;
+F2D_HD void warmStartCore(const ContactLane& c, const ContactMass& k, BodyState& bA, BodyState& bB) {
+  float tx = c.ny;
+  float ty = 0.0f - c.nx;
+  F2D_UNROLL2
   for (int p = 0; p < 2; ++p) {
-    const int o = p == 0 ? 0 : (CN_A2X - CN_A1X);
-    float rAx = c(CN_A1X + o, lane), rAy = c(CN_A1Y + o, lane);
-    float rBx = c(CN_B1X + o, lane), rBy = c(CN_B1Y + o, lane);
-    float ni = c(CN_NI1 + o, lane), ti = c(CN_TI1 + o, lane);
-    float Px = ni * nx + ti * tx;
-    float Py = ni * ny + ti * ty;
-    bA.w = bA.w - iA * (rAx * Py - rAy * Px);
-    bA.v.x = bA.v.x - mA * Px;
-    bA.v.y = bA.v.y - mA * Py;
-    bB.w = bB.w + iB * (rBx * Py - rBy * Px);
-    bB.v.x = bB.v.x + mB * Px;
-    bB.v.y = bB.v.y + mB * Py;
+    float Px = c.ni[p] * c.nx + c.ti[p] * tx;
+    float Py = c.ni[p] * c.ny + c.ti[p] * ty;
+    bA.w = bA.w - k.iA * (c.ax[p] * Py - c.ay[p] * Px);
+    bA.v.x = bA.v.x - k.mA * Px;
+    bA.v.y = bA.v.y - k.mA * Py;
+    bB.w = bB.w + k.iB * (c.bx[p] * Py - c.by[p] * Px);
+    bB.v.x = bB.v.x + k.mB * Px;
+    bB.v.y = bB.v.y + k.mB * Py;
   }
-  float ri = c(CN_ROLLING_IMPULSE, lane);
-  bA.w = bA.w - iA * ri;
-  bB.w = bB.w + iB * ri;
-  scatterVel(states, ia, bA);
-  scatterVel(states, ib, bB);
+  bA.w = bA.w - k.iA * c.rollingImpulse;
+  bB.w = bB.w + k.iB * c.rollingImpulse;
 }
 
-// b2SolveContactsTask lane, S/contact_solver.c:1729-1967 (useBias = solve, !useBias = relax)
-F2D_HD void solveLane(const Cons& c, long lane, BodyState* states, float inv_h, float minBiasVel, bool useBias) {
-  int ia = c.geti(CN_INDEX_A, lane), ib = c.geti(CN_INDEX_B, lane);
-  BodyState bA = gather(states, ia);
-  BodyState bB = gather(states, ib);
-  float mA = c(CN_INV_MASS_A, lane), mB = c(CN_INV_MASS_B, lane);
-  float iA = c(CN_INV_I_A, lane), iB = c(CN_INV_I_B, lane);
-  float nx = c(CN_NX, lane), ny = c(CN_NY, lane);
-  float biasRate, massScale, impulseScale;
-  if (useBias) {
-    biasRate = c(CN_BIAS_RATE, lane);
-    massScale = c(CN_MASS_SCALE, lane);
-    impulseScale = c(CN_IMPULSE_SCALE, lane);
-  } else {
-    biasRate = 0.0f;
-    massScale = 1.0f;
-    impulseScale = 0.0f;
-  }
+// b2SolveContactsTask lane, S/contact_solver.c:1729-1967; soft: the contact's softness
+// (solve) or {0, 1, 0} (relax)
+F2D_HD void solveCore(ContactLane& c, const ContactMass& k, BodyState& bA, BodyState& bB, float inv_h,
+                      float minBiasVel, Softness soft) {
+  const float mA = k.mA, iA = k.iA, mB = k.mB, iB = k.iB;
+  const float nx = c.nx, ny = c.ny;
   float totalNormalImpulse = 0.0f;
   float dpx = bB.dp.x - bA.dp.x;
   float dpy = bB.dp.y - bA.dp.y;
+  F2D_UNROLL2
   for (int p = 0; p < 2; ++p) {
-    const int o = p == 0 ? 0 : (CN_A2X - CN_A1X);
-    float rAx = c(CN_A1X + o, lane), rAy = c(CN_A1Y + o, lane);
-    float rBx = c(CN_B1X + o, lane), rBy = c(CN_B1Y + o, lane);
+    float rAx = c.ax[p], rAy = c.ay[p];
+    float rBx = c.bx[p], rBy = c.by[p];
     // moving anchors for current separation
     float rsAx = bA.dq.c * rAx - bA.dq.s * rAy;
     float rsAy = bA.dq.s * rAx + bA.dq.c * rAy;
@@ -207,22 +162,22 @@ F2D_HD void solveLane(const Cons& c, long lane, BodyState* states, float inv_h, 
     float rsBy = bB.dq.s * rBx + bB.dq.c * rBy;
     float dsx = dpx + (rsBx - rsAx);
     float dsy = dpy + (rsBy - rsAy);
-    float s = (nx * dsx + ny * dsy) + c(CN_BASE_SEP1 + o, lane);
+    float s = (nx * dsx + ny * dsy) + c.sep[p];
     bool mask = s > 0.0f;
     float specBias = s * inv_h;
-    float softBias = maxf(biasRate * s, minBiasVel);
+    float softBias = maxf(soft.biasRate * s, minBiasVel);
     float bias = mask ? specBias : softBias;
-    float pointMassScale = mask ? 1.0f : massScale;
-    float pointImpulseScale = mask ? 0.0f : impulseScale;
+    float pointMassScale = mask ? 1.0f : soft.massScale;
+    float pointImpulseScale = mask ? 0.0f : soft.impulseScale;
     float dvx = (bB.v.x - bB.w * rBy) - (bA.v.x - bA.w * rAy);
     float dvy = (bB.v.y + bB.w * rBx) - (bA.v.y + bA.w * rAx);
     float vn = dvx * nx + dvy * ny;
-    float ni = c(CN_NI1 + o, lane);
-    float negImpulse = c(CN_NM1 + o, lane) * (pointMassScale * (vn + bias)) + pointImpulseScale * ni;
+    float ni = c.ni[p];
+    float negImpulse = c.nm[p] * (pointMassScale * (vn + bias)) + pointImpulseScale * ni;
     float newImpulse = maxf(ni - negImpulse, 0.0f);
     float impulse = newImpulse - ni;
-    c(CN_NI1 + o, lane) = newImpulse;
-    c(CN_TNI1 + o, lane) = c(CN_TNI1 + o, lane) + newImpulse;
+    c.ni[p] = newImpulse;
+    c.tni[p] = c.tni[p] + newImpulse;
     totalNormalImpulse = totalNormalImpulse + newImpulse;
     float Px = impulse * nx;
     float Py = impulse * ny;
@@ -235,23 +190,21 @@ F2D_HD void solveLane(const Cons& c, long lane, BodyState* states, float inv_h, 
   }
   float tx = ny;
   float ty = 0.0f - nx;
-  float friction = c(CN_FRICTION, lane);
-  float tangentSpeed = c(CN_TANGENT_SPEED, lane);
+  F2D_UNROLL2
   for (int p = 0; p < 2; ++p) {
-    const int o = p == 0 ? 0 : (CN_A2X - CN_A1X);
-    float rAx = c(CN_A1X + o, lane), rAy = c(CN_A1Y + o, lane);
-    float rBx = c(CN_B1X + o, lane), rBy = c(CN_B1Y + o, lane);
+    float rAx = c.ax[p], rAy = c.ay[p];
+    float rBx = c.bx[p], rBy = c.by[p];
     float dvx = (bB.v.x - bB.w * rBy) - (bA.v.x - bA.w * rAy);
     float dvy = (bB.v.y + bB.w * rBx) - (bA.v.y + bA.w * rAx);
     float vt = dvx * tx + dvy * ty;
-    vt = vt - tangentSpeed;
-    float negImpulse = c(CN_TM1 + o, lane) * vt;
-    float maxFriction = friction * c(CN_NI1 + o, lane);
-    float ti = c(CN_TI1 + o, lane);
+    vt = vt - c.tangentSpeed;
+    float negImpulse = c.tm[p] * vt;
+    float maxFriction = c.friction * c.ni[p];
+    float ti = c.ti[p];
     float newImpulse = ti - negImpulse;
     newImpulse = maxf(0.0f - maxFriction, minf(newImpulse, maxFriction));
     float impulse = newImpulse - ti;
-    c(CN_TI1 + o, lane) = newImpulse;
+    c.ti[p] = newImpulse;
     float Px = impulse * tx;
     float Py = impulse * ty;
     bA.v.x = bA.v.x - mA * Px;
@@ -262,86 +215,70 @@ F2D_HD void solveLane(const Cons& c, long lane, BodyState* states, float inv_h, 
     bB.w = bB.w + iB * (rBx * Py - rBy * Px);
   }
   {
-    float deltaLambda = c(CN_ROLLING_MASS, lane) * (bA.w - bB.w);
-    float lambda = c(CN_ROLLING_IMPULSE, lane);
-    float maxLambda = c(CN_ROLLING_RES, lane) * totalNormalImpulse;
+    float deltaLambda = c.rollingMass * (bA.w - bB.w);
+    float lambda = c.rollingImpulse;
+    float maxLambda = c.rollingRes * totalNormalImpulse;
     // b2SymClampW: max(-b, min(a, b)) with -b formed by flipping the sign bit
     float a = lambda + deltaLambda;
     float nb = -maxLambda;
     float ri = maxf(nb, minf(a, maxLambda));
-    c(CN_ROLLING_IMPULSE, lane) = ri;
+    c.rollingImpulse = ri;
     deltaLambda = ri - lambda;
     bA.w = bA.w - iA * deltaLambda;
     bB.w = bB.w + iB * deltaLambda;
   }
-  scatterVel(states, ia, bA);
-  scatterVel(states, ib, bB);
 }
 
 // b2ApplyRestitutionTask lane, S/contact_solver.c:1969-2076. A lane with zero
-// restitution is skipped: in the 4-wide code such a lane is masked to zero mass,
-// which leaves its impulses and velocities unchanged.
-F2D_HD void restitutionLane(const Cons& c, long lane, BodyState* states, float threshold) {
-  float restitution = c(CN_RESTITUTION, lane);
-  if (restitution == 0.0f) return;
-  int ia = c.geti(CN_INDEX_A, lane), ib = c.geti(CN_INDEX_B, lane);
-  BodyState bA = gather(states, ia);
-  BodyState bB = gather(states, ib);
-  float mA = c(CN_INV_MASS_A, lane), mB = c(CN_INV_MASS_B, lane);
-  float iA = c(CN_INV_I_A, lane), iB = c(CN_INV_I_B, lane);
-  float nx = c(CN_NX, lane), ny = c(CN_NY, lane);
+// restitution is skipped by the callers: in the 4-wide code such a lane is masked to
+// zero mass, which leaves its impulses and velocities unchanged.
+F2D_HD void restitutionCore(ContactLane& c, const ContactMass& k, BodyState& bA, BodyState& bB, float restitution,
+                            const float* relVel, float threshold) {
+  F2D_UNROLL2
   for (int p = 0; p < 2; ++p) {
-    const int o = p == 0 ? 0 : (CN_A2X - CN_A1X);
-    const int rvf = p == 0 ? CN_REL_VEL1 : CN_REL_VEL2;
-    float relVel = c(rvf, lane);
-    bool mask1 = (relVel + threshold) > 0.0f;
-    bool mask2 = c(CN_TNI1 + o, lane) == 0.0f;
+    bool mask1 = (relVel[p] + threshold) > 0.0f;
+    bool mask2 = c.tni[p] == 0.0f;
     bool mask = mask1 || mask2;
-    float mass = mask ? 0.0f : c(CN_NM1 + o, lane);
-    float rAx = c(CN_A1X + o, lane), rAy = c(CN_A1Y + o, lane);
-    float rBx = c(CN_B1X + o, lane), rBy = c(CN_B1Y + o, lane);
+    float mass = mask ? 0.0f : c.nm[p];
+    float rAx = c.ax[p], rAy = c.ay[p];
+    float rBx = c.bx[p], rBy = c.by[p];
     float dvx = (bB.v.x - bB.w * rBy) - (bA.v.x - bA.w * rAy);
     float dvy = (bB.v.y + bB.w * rBx) - (bA.v.y + bA.w * rAx);
-    float vn = dvx * nx + dvy * ny;
-    float negImpulse = mass * (vn + restitution * relVel);
-    float ni = c(CN_NI1 + o, lane);
+    float vn = dvx * c.nx + dvy * c.ny;
+    float negImpulse = mass * (vn + restitution * relVel[p]);
+    float ni = c.ni[p];
     float newImpulse = maxf(ni - negImpulse, 0.0f);
     float impulse = newImpulse - ni;
-    c(CN_NI1 + o, lane) = newImpulse;
-    float Px = impulse * nx;
-    float Py = impulse * ny;
-    bA.v.x = bA.v.x - mA * Px;
-    bA.v.y = bA.v.y - mA * Py;
-    bA.w = bA.w - iA * (rAx * Py - rAy * Px);
-    bB.v.x = bB.v.x + mB * Px;
-    bB.v.y = bB.v.y + mB * Py;
-    bB.w = bB.w + iB * (rBx * Py - rBy * Px);
+    c.ni[p] = newImpulse;
+    float Px = impulse * c.nx;
+    float Py = impulse * c.ny;
+    bA.v.x = bA.v.x - k.mA * Px;
+    bA.v.y = bA.v.y - k.mA * Py;
+    bA.w = bA.w - k.iA * (rAx * Py - rAy * Px);
+    bB.v.x = bB.v.x + k.mB * Px;
+    bB.v.y = bB.v.y + k.mB * Py;
+    bB.w = bB.w + k.iB * (rBx * Py - rBy * Px);
   }
-  scatterVel(states, ia, bA);
-  scatterVel(states, ib, bB);
 }
 
 // b2StoreImpulsesTask lane, S/contact_solver.c:2078-2120 (writes both points)
-F2D_HD void storeLane(const Cons& c, long lane, Contact& cs) {
+F2D_HD void storeLane(const ContactLane& c, const float* relVel, Contact& cs) {
   Manifold& m = cs.m;
-  m.rollingImpulse = c(CN_ROLLING_IMPULSE, lane);
-  m.points[0].normalImpulse = c(CN_NI1, lane);
-  m.points[0].tangentImpulse = c(CN_TI1, lane);
-  m.points[0].totalNormalImpulse = c(CN_TNI1, lane);
-  m.points[0].normalVelocity = c(CN_REL_VEL1, lane);
-  m.points[1].normalImpulse = c(CN_NI2, lane);
-  m.points[1].tangentImpulse = c(CN_TI2, lane);
-  m.points[1].totalNormalImpulse = c(CN_TNI2, lane);
-  m.points[1].normalVelocity = c(CN_REL_VEL2, lane);
+  m.rollingImpulse = c.rollingImpulse;
+  F2D_UNROLL2
+  for (int p = 0; p < 2; ++p) {
+    m.points[p].normalImpulse = c.ni[p];
+    m.points[p].tangentImpulse = c.ti[p];
+    m.points[p].totalNormalImpulse = c.tni[p];
+    m.points[p].normalVelocity = relVel[p];
+  }
 }
 
-// ---------------------------------------------------------------------------- overflow (scalar order)
+// ---------------------------------------------------------------------------- lanes in memory
 
-// Static bodies have no solver state: the scalar solver reads and writes a dummy
-// identity state for them (S/contact_solver.c:175-176). Their inverse mass and
-// inertia are zero, so for finite impulses the dummy's velocities stay exactly +0
-// and its deltas the identity; reading the identity and dropping the write is
-// therefore the same computation.
+// Static bodies have no solver state: they read the identity state and drop the write
+// (S/contact_solver.c:175-176; their inverse mass and inertia are zero, so the scalar
+// solver's dummy state never changes either).
 F2D_HD BodyState loadState(const BodyState* states, int idx) { return idx < 0 ? identityState() : states[idx]; }
 F2D_HD void storeVel(BodyState* states, int idx, Vec2 v, float w) {
   if (idx >= 0) {
@@ -350,42 +287,138 @@ F2D_HD void storeVel(BodyState* states, int idx, Vec2 v, float w) {
   }
 }
 
+// Every field that the solve stages read, loaded together (the loads are issued back to
+// back, before the first store of the stage)
+F2D_HD void loadLane(const Cons& c, long lane, int4& head, ContactLane& l, ContactMass& k) {
+  const float4 g0 = c.group(0, lane), g1 = c.group(1, lane), g2 = c.group(2, lane), g3 = c.group(3, lane),
+               g4 = c.group(4, lane), g5 = c.group(5, lane), g6 = c.group(6, lane), g7 = c.group(7, lane),
+               g8 = c.group(8, lane);
+  head = make_int4(asInt(g0.x), asInt(g0.y), asInt(g0.z), asInt(g0.w));
+  l.nx = g1.x, l.ny = g1.y, l.friction = g1.z, l.tangentSpeed = g1.w;
+  l.ax[0] = g2.x, l.ay[0] = g2.y, l.bx[0] = g2.z, l.by[0] = g2.w;
+  l.ax[1] = g3.x, l.ay[1] = g3.y, l.bx[1] = g3.z, l.by[1] = g3.w;
+  l.sep[0] = g4.x, l.sep[1] = g4.y, l.nm[0] = g4.z, l.nm[1] = g4.w;
+  l.tm[0] = g5.x, l.tm[1] = g5.y, l.rollingRes = g5.z, l.rollingMass = g5.w;
+  l.ni[0] = g6.x, l.ti[0] = g6.y, l.ni[1] = g6.z, l.ti[1] = g6.w;
+  l.tni[0] = g7.x, l.tni[1] = g7.y, l.rollingImpulse = g7.z;
+  k.mA = g8.x, k.iA = g8.y, k.mB = g8.z, k.iB = g8.w;
+}
+F2D_HD void storeLaneImpulses(const Cons& c, long lane, const ContactLane& l) {
+  c.group(6, lane) = make_float4(l.ni[0], l.ti[0], l.ni[1], l.ti[1]);
+  c.group(7, lane) = make_float4(l.tni[0], l.tni[1], l.rollingImpulse, 0.0f);
+}
+
+// indexA, indexB: solver state of each body, -1 for a static one
+F2D_HD void prepareMemoryLane(const Cons& c, long lane, const Contact& cs, int slot, int indexA, int indexB,
+                              const ContactMass& k, const BodyState* states, float warmStartScale) {
+  ContactLane l;
+  float relVel[2];
+  prepareLane(l, cs, k, loadState(states, indexA), loadState(states, indexB), warmStartScale, relVel);
+  c.group(0, lane) = make_float4(asFloat(indexA), asFloat(indexB), asFloat(slot), asFloat(cs.m.pointCount));
+  c.group(1, lane) = make_float4(l.nx, l.ny, l.friction, l.tangentSpeed);
+  c.group(2, lane) = make_float4(l.ax[0], l.ay[0], l.bx[0], l.by[0]);
+  c.group(3, lane) = make_float4(l.ax[1], l.ay[1], l.bx[1], l.by[1]);
+  c.group(4, lane) = make_float4(l.sep[0], l.sep[1], l.nm[0], l.nm[1]);
+  c.group(5, lane) = make_float4(l.tm[0], l.tm[1], l.rollingRes, l.rollingMass);
+  storeLaneImpulses(c, lane, l);
+  c.group(8, lane) = make_float4(k.mA, k.iA, k.mB, k.iB);
+  c.group(9, lane) = make_float4(cs.restitution, relVel[0], relVel[1], 0.0f);
+}
+
+F2D_HD void warmStartMemoryLane(const Cons& c, long lane, BodyState* states) {
+  int4 head;
+  ContactLane l;
+  ContactMass k;
+  loadLane(c, lane, head, l, k);
+  BodyState bA = loadState(states, head.x), bB = loadState(states, head.y);
+  warmStartCore(l, k, bA, bB);
+  storeVel(states, head.x, bA.v, bA.w);
+  storeVel(states, head.y, bB.v, bB.w);
+}
+
+// contactSoft, staticSoft: the softness between two bodies and against a static one
+F2D_HD void solveMemoryLane(const Cons& c, long lane, BodyState* states, float inv_h, float minBiasVel, bool useBias,
+                            Softness contactSoft, Softness staticSoft) {
+  int4 head;
+  ContactLane l;
+  ContactMass k;
+  loadLane(c, lane, head, l, k);
+  BodyState bA = loadState(states, head.x), bB = loadState(states, head.y);
+  const Softness relax = {0.0f, 1.0f, 0.0f};
+  solveCore(l, k, bA, bB, inv_h, minBiasVel, useBias ? ((head.x < 0 || head.y < 0) ? staticSoft : contactSoft) : relax);
+  storeLaneImpulses(c, lane, l);
+  storeVel(states, head.x, bA.v, bA.w);
+  storeVel(states, head.y, bB.v, bB.w);
+}
+
+F2D_HD void restitutionMemoryLane(const Cons& c, long lane, BodyState* states, float threshold) {
+  const float4 g9 = c.group(9, lane);
+  if (g9.x == 0.0f) return;
+  const float relVel[2] = {g9.y, g9.z};
+  int4 head;
+  ContactLane l;
+  ContactMass k;
+  loadLane(c, lane, head, l, k);
+  BodyState bA = loadState(states, head.x), bB = loadState(states, head.y);
+  restitutionCore(l, k, bA, bB, g9.x, relVel, threshold);
+  storeLaneImpulses(c, lane, l);
+  storeVel(states, head.x, bA.v, bA.w);
+  storeVel(states, head.y, bB.v, bB.w);
+}
+
+F2D_HD void storeMemoryLane(const Cons& c, long lane, Contact& cs) {
+  int4 head;
+  ContactLane l;
+  ContactMass k;
+  loadLane(c, lane, head, l, k);
+  const float4 g9 = c.group(9, lane);
+  const float relVel[2] = {g9.y, g9.z};
+  storeLane(l, relVel, cs);
+}
+
+// ---------------------------------------------------------------------------- overflow (scalar order)
+
 // b2WarmStartOverflowContacts body, S/contact_solver.c:160-225
 F2D_HD void overflowWarmStart(const Cons& c, long lane, BodyState* states) {
-  int ia = c.geti(CN_INDEX_A, lane), ib = c.geti(CN_INDEX_B, lane);
+  int4 head;
+  ContactLane l;
+  ContactMass k;
+  loadLane(c, lane, head, l, k);
+  const int ia = head.x, ib = head.y, pointCount = head.w;
   BodyState sA = loadState(states, ia);
   BodyState sB = loadState(states, ib);
   Vec2 vA = sA.v;
   float wA = sA.w;
   Vec2 vB = sB.v;
   float wB = sB.w;
-  float mA = c(CN_INV_MASS_A, lane), iA = c(CN_INV_I_A, lane);
-  float mB = c(CN_INV_MASS_B, lane), iB = c(CN_INV_I_B, lane);
-  Vec2 normal = {c(CN_NX, lane), c(CN_NY, lane)};
+  Vec2 normal = {l.nx, l.ny};
   Vec2 tangent = rightPerp(normal);
-  int pointCount = c.geti(CN_POINT_COUNT, lane);
-  for (int p = 0; p < pointCount; ++p) {
-    const int o = p == 0 ? 0 : (CN_A2X - CN_A1X);
-    Vec2 rA = {c(CN_A1X + o, lane), c(CN_A1Y + o, lane)};
-    Vec2 rB = {c(CN_B1X + o, lane), c(CN_B1Y + o, lane)};
-    Vec2 P = add(mulSV(c(CN_NI1 + o, lane), normal), mulSV(c(CN_TI1 + o, lane), tangent));
-    wA -= iA * cross(rA, P);
-    vA = mulAdd(vA, -mA, P);
-    wB += iB * cross(rB, P);
-    vB = mulAdd(vB, mB, P);
+  F2D_UNROLL2
+  for (int p = 0; p < 2; ++p) {
+    if (p >= pointCount) break;
+    Vec2 rA = {l.ax[p], l.ay[p]};
+    Vec2 rB = {l.bx[p], l.by[p]};
+    Vec2 P = add(mulSV(l.ni[p], normal), mulSV(l.ti[p], tangent));
+    wA -= k.iA * cross(rA, P);
+    vA = mulAdd(vA, -k.mA, P);
+    wB += k.iB * cross(rB, P);
+    vB = mulAdd(vB, k.mB, P);
   }
-  float ri = c(CN_ROLLING_IMPULSE, lane);
-  wA -= iA * ri;
-  wB += iB * ri;
+  wA -= k.iA * l.rollingImpulse;
+  wB += k.iB * l.rollingImpulse;
   storeVel(states, ia, vA, wA);
   storeVel(states, ib, vB, wB);
 }
 
 // b2SolveOverflowContacts body, S/contact_solver.c:227-380
-F2D_HD void overflowSolve(const Cons& c, long lane, BodyState* states, float inv_h, float pushout, bool useBias) {
-  float mA = c(CN_INV_MASS_A, lane), iA = c(CN_INV_I_A, lane);
-  float mB = c(CN_INV_MASS_B, lane), iB = c(CN_INV_I_B, lane);
-  int ia = c.geti(CN_INDEX_A, lane), ib = c.geti(CN_INDEX_B, lane);
+F2D_HD void overflowSolve(const Cons& c, long lane, BodyState* states, float inv_h, float pushout, bool useBias,
+                          Softness contactSoft, Softness staticSoft) {
+  int4 head;
+  ContactLane l;
+  ContactMass k;
+  loadLane(c, lane, head, l, k);
+  const int ia = head.x, ib = head.y, pointCount = head.w;
+  const float mA = k.mA, iA = k.iA, mB = k.mB, iB = k.iB;
   BodyState sA = loadState(states, ia);
   Vec2 vA = sA.v;
   float wA = sA.w;
@@ -395,18 +428,17 @@ F2D_HD void overflowSolve(const Cons& c, long lane, BodyState* states, float inv
   float wB = sB.w;
   Rot dqB = sB.dq;
   Vec2 dp = sub(sB.dp, sA.dp);
-  Vec2 normal = {c(CN_NX, lane), c(CN_NY, lane)};
+  Vec2 normal = {l.nx, l.ny};
   Vec2 tangent = rightPerp(normal);
-  float friction = c(CN_FRICTION, lane);
-  Softness softness = {c(CN_BIAS_RATE, lane), c(CN_MASS_SCALE, lane), c(CN_IMPULSE_SCALE, lane)};
-  int pointCount = c.geti(CN_POINT_COUNT, lane);
+  Softness softness = (ia < 0 || ib < 0) ? staticSoft : contactSoft;
   float totalNormalImpulse = 0.0f;
-  for (int p = 0; p < pointCount; ++p) {
-    const int o = p == 0 ? 0 : (CN_A2X - CN_A1X);
-    Vec2 rA = {c(CN_A1X + o, lane), c(CN_A1Y + o, lane)};
-    Vec2 rB = {c(CN_B1X + o, lane), c(CN_B1Y + o, lane)};
+  F2D_UNROLL2
+  for (int p = 0; p < 2; ++p) {
+    if (p >= pointCount) break;
+    Vec2 rA = {l.ax[p], l.ay[p]};
+    Vec2 rB = {l.bx[p], l.by[p]};
     Vec2 ds = add(dp, sub(rotate(dqB, rB), rotate(dqA, rA)));
-    float s = c(CN_BASE_SEP1 + o, lane) + dot(ds, normal);
+    float s = l.sep[p] + dot(ds, normal);
     float velocityBias = 0.0f;
     float massScale = 1.0f;
     float impulseScale = 0.0f;
@@ -420,12 +452,12 @@ F2D_HD void overflowSolve(const Cons& c, long lane, BodyState* states, float inv
     Vec2 vrA = add(vA, crossSV(wA, rA));
     Vec2 vrB = add(vB, crossSV(wB, rB));
     float vn = dot(sub(vrB, vrA), normal);
-    float ni = c(CN_NI1 + o, lane);
-    float impulse = -c(CN_NM1 + o, lane) * massScale * (vn + velocityBias) - impulseScale * ni;
+    float ni = l.ni[p];
+    float impulse = -l.nm[p] * massScale * (vn + velocityBias) - impulseScale * ni;
     float newImpulse = maxf(ni + impulse, 0.0f);
     impulse = newImpulse - ni;
-    c(CN_NI1 + o, lane) = newImpulse;
-    c(CN_TNI1 + o, lane) = c(CN_TNI1 + o, lane) + newImpulse;
+    l.ni[p] = newImpulse;
+    l.tni[p] = l.tni[p] + newImpulse;
     totalNormalImpulse += newImpulse;
     Vec2 P = mulSV(impulse, normal);
     vA = mulSub(vA, mA, P);
@@ -433,20 +465,20 @@ F2D_HD void overflowSolve(const Cons& c, long lane, BodyState* states, float inv
     vB = mulAdd(vB, mB, P);
     wB += iB * cross(rB, P);
   }
-  float tangentSpeed = c(CN_TANGENT_SPEED, lane);
-  for (int p = 0; p < pointCount; ++p) {
-    const int o = p == 0 ? 0 : (CN_A2X - CN_A1X);
-    Vec2 rA = {c(CN_A1X + o, lane), c(CN_A1Y + o, lane)};
-    Vec2 rB = {c(CN_B1X + o, lane), c(CN_B1Y + o, lane)};
+  F2D_UNROLL2
+  for (int p = 0; p < 2; ++p) {
+    if (p >= pointCount) break;
+    Vec2 rA = {l.ax[p], l.ay[p]};
+    Vec2 rB = {l.bx[p], l.by[p]};
     Vec2 vrB = add(vB, crossSV(wB, rB));
     Vec2 vrA = add(vA, crossSV(wA, rA));
-    float vt = dot(sub(vrB, vrA), tangent) - tangentSpeed;
-    float impulse = c(CN_TM1 + o, lane) * (-vt);
-    float maxFriction = friction * c(CN_NI1 + o, lane);
-    float ti = c(CN_TI1 + o, lane);
+    float vt = dot(sub(vrB, vrA), tangent) - l.tangentSpeed;
+    float impulse = l.tm[p] * (-vt);
+    float maxFriction = l.friction * l.ni[p];
+    float ti = l.ti[p];
     float newImpulse = clampf(ti + impulse, -maxFriction, maxFriction);
     impulse = newImpulse - ti;
-    c(CN_TI1 + o, lane) = newImpulse;
+    l.ti[p] = newImpulse;
     Vec2 P = mulSV(impulse, tangent);
     vA = mulSub(vA, mA, P);
     wA -= iA * cross(rA, P);
@@ -454,56 +486,60 @@ F2D_HD void overflowSolve(const Cons& c, long lane, BodyState* states, float inv
     wB += iB * cross(rB, P);
   }
   {
-    float deltaLambda = -c(CN_ROLLING_MASS, lane) * (wB - wA);
-    float lambda = c(CN_ROLLING_IMPULSE, lane);
-    float maxLambda = c(CN_ROLLING_RES, lane) * totalNormalImpulse;
+    float deltaLambda = -l.rollingMass * (wB - wA);
+    float lambda = l.rollingImpulse;
+    float maxLambda = l.rollingRes * totalNormalImpulse;
     float ri = clampf(lambda + deltaLambda, -maxLambda, maxLambda);
-    c(CN_ROLLING_IMPULSE, lane) = ri;
+    l.rollingImpulse = ri;
     deltaLambda = ri - lambda;
     wA -= iA * deltaLambda;
     wB += iB * deltaLambda;
   }
+  storeLaneImpulses(c, lane, l);
   storeVel(states, ia, vA, wA);
   storeVel(states, ib, vB, wB);
 }
 
 // b2ApplyOverflowRestitution body, S/contact_solver.c:382-478
 F2D_HD void overflowRestitution(const Cons& c, long lane, BodyState* states, float threshold) {
-  float restitution = c(CN_RESTITUTION, lane);
+  const float4 g9 = c.group(9, lane);
+  const float restitution = g9.x;
   if (restitution == 0.0f) return;
-  float mA = c(CN_INV_MASS_A, lane), iA = c(CN_INV_I_A, lane);
-  float mB = c(CN_INV_MASS_B, lane), iB = c(CN_INV_I_B, lane);
-  int ia = c.geti(CN_INDEX_A, lane), ib = c.geti(CN_INDEX_B, lane);
+  int4 head;
+  ContactLane l;
+  ContactMass k;
+  loadLane(c, lane, head, l, k);
+  const int ia = head.x, ib = head.y, pointCount = head.w;
   BodyState sA = loadState(states, ia);
   Vec2 vA = sA.v;
   float wA = sA.w;
   BodyState sB = loadState(states, ib);
   Vec2 vB = sB.v;
   float wB = sB.w;
-  Vec2 normal = {c(CN_NX, lane), c(CN_NY, lane)};
-  int pointCount = c.geti(CN_POINT_COUNT, lane);
-  for (int p = 0; p < pointCount; ++p) {
-    const int o = p == 0 ? 0 : (CN_A2X - CN_A1X);
-    const int rvf = p == 0 ? CN_REL_VEL1 : CN_REL_VEL2;
-    float relVel = c(rvf, lane);
-    if (relVel > -threshold || c(CN_TNI1 + o, lane) == 0.0f) continue;
-    Vec2 rA = {c(CN_A1X + o, lane), c(CN_A1Y + o, lane)};
-    Vec2 rB = {c(CN_B1X + o, lane), c(CN_B1Y + o, lane)};
+  Vec2 normal = {l.nx, l.ny};
+  F2D_UNROLL2
+  for (int p = 0; p < 2; ++p) {
+    if (p >= pointCount) break;
+    float relVel = p == 0 ? g9.y : g9.z;
+    if (relVel > -threshold || l.tni[p] == 0.0f) continue;
+    Vec2 rA = {l.ax[p], l.ay[p]};
+    Vec2 rB = {l.bx[p], l.by[p]};
     Vec2 vrB = add(vB, crossSV(wB, rB));
     Vec2 vrA = add(vA, crossSV(wA, rA));
     float vn = dot(sub(vrB, vrA), normal);
-    float impulse = -c(CN_NM1 + o, lane) * (vn + restitution * relVel);
-    float ni = c(CN_NI1 + o, lane);
+    float impulse = -l.nm[p] * (vn + restitution * relVel);
+    float ni = l.ni[p];
     float newImpulse = maxf(ni + impulse, 0.0f);
     impulse = newImpulse - ni;
-    c(CN_NI1 + o, lane) = newImpulse;
-    c(CN_TNI1 + o, lane) = c(CN_TNI1 + o, lane) + impulse;
+    l.ni[p] = newImpulse;
+    l.tni[p] = l.tni[p] + impulse;
     Vec2 P = mulSV(impulse, normal);
-    vA = mulSub(vA, mA, P);
-    wA -= iA * cross(rA, P);
-    vB = mulAdd(vB, mB, P);
-    wB += iB * cross(rB, P);
+    vA = mulSub(vA, k.mA, P);
+    wA -= k.iA * cross(rA, P);
+    vB = mulAdd(vB, k.mB, P);
+    wB += k.iB * cross(rB, P);
   }
+  storeLaneImpulses(c, lane, l);
   storeVel(states, ia, vA, wA);
   storeVel(states, ib, vB, wB);
 }
@@ -511,15 +547,20 @@ F2D_HD void overflowRestitution(const Cons& c, long lane, BodyState* states, flo
 // b2StoreOverflowImpulses body, S/contact_solver.c:480-509 (writes pointCount points)
 F2D_HD void overflowStore(const Cons& c, long lane, Contact& cs) {
   Manifold& m = cs.m;
-  for (int p = 0; p < m.pointCount; ++p) {
-    const int o = p == 0 ? 0 : (CN_A2X - CN_A1X);
-    const int rvf = p == 0 ? CN_REL_VEL1 : CN_REL_VEL2;
-    m.points[p].normalImpulse = c(CN_NI1 + o, lane);
-    m.points[p].tangentImpulse = c(CN_TI1 + o, lane);
-    m.points[p].totalNormalImpulse = c(CN_TNI1 + o, lane);
-    m.points[p].normalVelocity = c(rvf, lane);
+  int4 head;
+  ContactLane l;
+  ContactMass k;
+  loadLane(c, lane, head, l, k);
+  const float4 g9 = c.group(9, lane);
+  F2D_UNROLL2
+  for (int p = 0; p < 2; ++p) {
+    if (p >= m.pointCount) break;
+    m.points[p].normalImpulse = l.ni[p];
+    m.points[p].tangentImpulse = l.ti[p];
+    m.points[p].totalNormalImpulse = l.tni[p];
+    m.points[p].normalVelocity = p == 0 ? g9.y : g9.z;
   }
-  m.rollingImpulse = c(CN_ROLLING_IMPULSE, lane);
+  m.rollingImpulse = l.rollingImpulse;
 }
 
 // ---------------------------------------------------------------------------- bodies
@@ -561,8 +602,8 @@ struct alignas(16) BodyConst {
   Vec2 dv;        // h*invMass*force + h*gravityScale*gravity
   float dw;       // h*invI*torque
   float linDamp;  // 1 / (1 + h*linearDamping)
+  float invMass, invI;  // one 8-byte access
   float angDamp;  // 1 / (1 + h*angularDamping)
-  float invMass, invI;
   int flags;      // BC_*
 };
 

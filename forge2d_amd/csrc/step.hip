@@ -53,6 +53,9 @@ struct SharedState {
   int error;
   int pairCount;
   int noAwake;  // no awake body: b2Solve returns after merging islands
+  int otherJoints;  // a joint of another type than revolute
+  int stageCount;   // colours with constraints below, in order
+  int4 stages[kOverflowIndex];  // first contact lane, contacts, first joint, joints
 };
 
 // Sweeps of shapes whose x-range covers many others (ground and ceiling segments),
@@ -211,7 +214,7 @@ __device__ WorldPtrs worldPtrs(const BatchView& b, WorldHeader* h) {
   w.colorBits = b.colorBits + h->colorOffset;
   w.overflow = b.overflow + h->overflowOffset;
   w.colorLists = b.colorLists + h->colorListOffset;
-  w.cons.f = b.cons + h->constraintOffset;
+  w.cons.f = b.cons + 4L * h->constraintOffset;
   w.cons.stride = b.consStride;
   w.scratch = b.scratch + h->scratchOffset;
   w.ccolor = b.ccolor + h->contactOffset;
@@ -1227,177 +1230,566 @@ struct SolveCtx {
   bool enableContinuous, enableSleep;
 };
 
+// b2Solve, S/solver.c:1190-1220 and :1479-1706: merge islands linked since the last
+// step, stop when no body is awake (returns false), split the last step's candidate
+// island.
+//
+// b2MergeAwakeIslands (S/island.c:547-590): its first loop leaves every awake island
+// pointing at its root; here every lane walks its islands' parent chains read-only (a
+// chain read while other lanes shorten it still ends at the same root) and writes its
+// own island's root, then one lane merges in reverse awake order.
+template <int BLOCK>
+__device__ __forceinline__ bool solveIslands(const WorldPtrs& w, SharedState& sh) {
+  WorldHeader* h = w.hdr;
+  const int nb = h->bodyCount, nc = h->contactCount;
+  const bool merge = h->mergePending != 0;
+  if (merge) {
+    IslandCtx ic = w.isl;
+    for (int i = threadIdx.x; i < h->awakeIslandCount; i += BLOCK) {
+      const int id = ic.awakeIslands[i];
+      int root = id;
+      for (int guard = h->islandCount; ic.islands[root].parent != -1 && guard > 0; --guard)
+        root = ic.islands[root].parent;
+      if (root != id) ic.islands[id].parent = root;
+    }
+    __syncthreads();
+    // the relabelling of b2MergeIsland on all lanes: whatever belongs to an awake
+    // island with a parent (a child to merge) takes the parent's (its root's) id
+    const int ni = h->islandCap;
+    for (int i = threadIdx.x; i < nb; i += BLOCK) {
+      const int id = w.sims[i].islandId;
+      if (id < 0 || id >= ni) continue;
+      const Island& is = ic.islands[id];
+      if (is.parent != -1 && is.setIndex == kAwakeSet) w.sims[i].islandId = is.parent;
+    }
+    for (int k = threadIdx.x; k < nc; k += BLOCK) {
+      const int id = w.links[k].x;
+      if (id < 0 || id >= ni) continue;
+      const Island& is = ic.islands[id];
+      if (is.parent != -1 && is.setIndex == kAwakeSet) w.links[k].x = is.parent;
+    }
+    for (int j = threadIdx.x; j < h->jointCount; j += BLOCK) {
+      const int id = w.joints[j].islandId;
+      if (id < 0 || id >= ni) continue;
+      const Island& is = ic.islands[id];
+      if (is.parent != -1 && is.setIndex == kAwakeSet) w.joints[j].islandId = is.parent;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    IslandCtx ic = w.isl;
+    if (merge) mergeAwakeChildren(ic);
+    sh.noAwake = h->awakeBodyCount == 0 ? 1 : 0;
+    if (!sh.noAwake && h->splitIslandId != -1) splitIsland(ic, h->splitIslandId);
+    if (!sh.noAwake) h->splitIslandId = -1;
+  }
+  __syncthreads();
+  return sh.noAwake == 0;
+}
+
+// The touching contacts by colour are the colour arrays; the joints by colour are
+// counted here. Fills the counts and starts (overflow last) and the list of colours
+// that have constraints.
+template <int BLOCK>
+__device__ __forceinline__ void solveColors(const WorldPtrs& w, SharedState& sh) {
+  WorldHeader* h = w.hdr;
+  if (threadIdx.x < kGraphColorCount) {
+    sh.colorCount[threadIdx.x] = threadIdx.x < kOverflowIndex ? w.colorLists[threadIdx.x] : h->overflowCount;
+    sh.jointColorCount[threadIdx.x] = 0;
+    sh.jointColorFill[threadIdx.x] = 0;
+    if (threadIdx.x == 0) sh.otherJoints = 0;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < h->jointCount; i += BLOCK) {
+    const Joint& j = w.joints[i];
+    if (j.color >= 0) atomicAdd(&sh.jointColorCount[j.color], 1);
+    if (j.type != kRevoluteJoint) sh.otherJoints = 1;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int s = 0, sj = 0, active = 0;
+    F2D_UNROLL
+    for (int k = 0; k < kOverflowIndex; ++k) {
+      const int n = sh.colorCount[k], nj = sh.jointColorCount[k];
+      sh.colorStart[k] = s;
+      sh.jointColorStart[k] = sj;
+      if (n + nj > 0) sh.stages[active++] = make_int4(s, n, sj, nj);
+      s += n;
+      sj += nj;
+    }
+    sh.colorStart[kOverflowIndex] = s;
+    sh.colorStart[kGraphColorCount] = s + sh.colorCount[kOverflowIndex];
+    sh.jointColorStart[kOverflowIndex] = sj;
+    sh.stageCount = active;
+    h->activeColors = active;
+  }
+  __syncthreads();
+}
+
+// Contact slot of contact lane `lane` (below the overflow lanes): its colour's array entry
+__device__ __forceinline__ int colorLaneSlot(const WorldPtrs& w, const SharedState& sh, int lane) {
+  int c = 0;
+  F2D_UNROLL
+  for (int k = 1; k < kOverflowIndex; ++k) c += lane >= sh.colorStart[k] ? 1 : 0;
+  // an empty colour starts where the next one does: the last colour that starts at or
+  // before the lane is the one that holds it
+  return w.colorLists[kColorListHeader + (long)c * w.hdr->bodyCount + (lane - sh.colorStart[c])];
+}
+
+// Joint ids by colour; the overflow's in its array order.
+template <int BLOCK>
+__device__ __forceinline__ void listJoints(const WorldPtrs& w, SharedState& sh, int* jointLanes) {
+  WorldHeader* h = w.hdr;
+  for (int i = threadIdx.x; i < h->jointCount; i += BLOCK) {
+    const Joint& j = w.joints[i];
+    if (j.color >= 0 && j.color < kOverflowIndex)
+      jointLanes[sh.jointColorStart[j.color] + atomicAdd(&sh.jointColorFill[j.color], 1)] = i;
+  }
+  if (threadIdx.x == 0 && sh.jointColorCount[kOverflowIndex] > 0) {
+    // overflow joints are solved one after another in their colour's array order
+    int* list = jointLanes + sh.jointColorStart[kOverflowIndex];
+    const int n = sh.jointColorCount[kOverflowIndex];
+    for (int k = 0; k < n; ++k) list[k] = -1;
+    for (int i = 0; i < h->jointCount; ++i) {
+      const Joint& j = w.joints[i];
+      if (j.color == kOverflowIndex && j.localIndex >= 0 && j.localIndex < n) list[j.localIndex] = i;
+    }
+    for (int k = 0; k < n; ++k)
+      if (list[k] < 0) h->error |= ERR_OVERFLOW_CAP;
+  }
+}
+
+// Contact lanes a lane of the resident solve keeps in registers: three (84 VGPRs of the
+// 128 that leave four wavefronts a SIMD), so a workgroup holds three contacts a lane.
+constexpr int kResidentLanes = 3;
+
+// The solver stages of a world whose contacts fit the workgroup's registers
+// (kResidentLanes x BLOCK lanes, no overflow) and whose bodies and revolute joints fit
+// LDS. A contact's terms are computed into registers by prepare and stay there until its
+// impulses are stored; a colour stage then touches LDS only for the two bodies. What
+// bounds it is the chain of one contact's arithmetic per colour, 4 x (2 x colours + 1)
+// times a step. The slot behind the bodies stands for every static body: identity state,
+// zero mass, never written.
+template <int BLOCK>
+__device__ __forceinline__ void solveResident(const WorldPtrs& w, SharedState& sh, BodyState* states,
+                                              BodyConst* consts, Joint* jts, const int* jointLanes,
+                                              const SolveCtx& ctx) {
+  const WorldHeader* h = w.hdr;
+  const int nb = h->bodyCount, t = threadIdx.x;
+  const int lanes = sh.colorStart[kOverflowIndex];
+  const int stageCount = __builtin_amdgcn_readfirstlane(sh.stageCount);
+  ContactLane cl[kResidentLanes];
+  int bodies[kResidentLanes];
+  auto loadBodies = [&](int j, BodyState& bA, BodyState& bB, ContactMass& k) {
+    const int ia = bodies[j] & 0xFFFF, ib = (int)((unsigned)bodies[j] >> 16);
+    bA = states[ia];
+    bB = states[ib];
+    k.mA = consts[ia].invMass, k.iA = consts[ia].invI;
+    k.mB = consts[ib].invMass, k.iB = consts[ib].invI;
+  };
+  auto storeBodies = [&](int j, const BodyState& bA, const BodyState& bB) {
+    const int ia = bodies[j] & 0xFFFF, ib = (int)((unsigned)bodies[j] >> 16);
+    if (ia != nb) {
+      states[ia].v = bA.v;
+      states[ia].w = bA.w;
+    }
+    if (ib != nb) {
+      states[ib].v = bB.v;
+      states[ib].w = bB.w;
+    }
+  };
+  // prepare joints, S/solver.c:967-987 -> S/joint.c:1348-1402
+  for (int i = t; i < h->jointCount; i += BLOCK) {
+    if (jts[i].color >= 0) prepareRevolute(jts[i], w.sims, ctx.h, ctx.inv_h, ctx.warmStartScale);
+  }
+  // prepare contacts; what only restitution and the store need waits in HBM
+  int restitution = 0;
+  F2D_UNROLL
+  for (int j = 0; j < kResidentLanes; ++j) {
+    const int lane = j * BLOCK + t;
+    bodies[j] = nb | (nb << 16);
+    if (lane >= lanes) continue;
+    const int slot = colorLaneSlot(w, sh, lane);
+    const Contact& c = w.contacts[slot];
+    const int ia = (consts[c.bodyA].flags & BC_STATIC) ? nb : c.bodyA;
+    const int ib = (consts[c.bodyB].flags & BC_STATIC) ? nb : c.bodyB;
+    bodies[j] = ia | (ib << 16);
+    BodyState bA, bB;
+    ContactMass k;
+    loadBodies(j, bA, bB, k);
+    float relVel[2];
+    prepareLane(cl[j], c, k, bA, bB, ctx.warmStartScale, relVel);
+    w.cons.group(0, lane) = make_float4(c.restitution, relVel[0], relVel[1], __int_as_float(slot));
+    restitution |= c.restitution != 0.0f ? 1 : 0;
+  }
+  restitution = __syncthreads_or(restitution);
+
+  auto warmStart = [&](int a) {
+    const int4 st = sh.stages[a];
+    for (int k = t; k < st.w; k += BLOCK) warmStartRevolute(jts[jointLanes[st.z + k]], states);
+    F2D_UNROLL
+    for (int j = 0; j < kResidentLanes; ++j) {
+      if ((unsigned)(j * BLOCK + t - st.x) < (unsigned)st.y) {
+        BodyState bA, bB;
+        ContactMass k;
+        loadBodies(j, bA, bB, k);
+        warmStartCore(cl[j], k, bA, bB);
+        storeBodies(j, bA, bB);
+      }
+    }
+    __syncthreads();
+  };
+  auto solve = [&](int a, bool useBias) {
+    const int4 st = sh.stages[a];
+    for (int k = t; k < st.w; k += BLOCK) solveRevolute(jts[jointLanes[st.z + k]], states, ctx.h, ctx.inv_h, useBias);
+    F2D_UNROLL
+    for (int j = 0; j < kResidentLanes; ++j) {
+      if ((unsigned)(j * BLOCK + t - st.x) < (unsigned)st.y) {
+        BodyState bA, bB;
+        ContactMass k;
+        loadBodies(j, bA, bB, k);
+        const bool fixed = (bodies[j] & 0xFFFF) == nb || (int)((unsigned)bodies[j] >> 16) == nb;
+        Softness soft = {0.0f, 1.0f, 0.0f};
+        if (useBias) soft = fixed ? ctx.staticSoftness : ctx.contactSoftness;
+        solveCore(cl[j], k, bA, bB, ctx.inv_h, -ctx.contactSpeed, soft);
+        storeBodies(j, bA, bB);
+      }
+    }
+    __syncthreads();
+  };
+  for (int sub = 0; sub < ctx.subSteps; ++sub) {
+    for (int i = t; i < nb; i += BLOCK) {
+      BodyConst k = consts[i];
+      if (k.flags & BC_STATIC) continue;
+      BodyState st = states[i];
+      integrateVelocityConst(k, st, ctx.maxLinearSpeed, ctx.maxAngularSpeed);
+      states[i] = st;
+      if (k.flags & BC_CAPPED) w.sims[i].flags |= BF_CAPPED_STEP;
+    }
+    __syncthreads();
+    for (int a = 0; a < stageCount; ++a) warmStart(a);
+    for (int pass = 0; pass < 2; ++pass) {
+      // solve, integrate positions, relax: one body of code for solve and relax
+      for (int a = 0; a < stageCount; ++a) solve(a, pass == 0);
+      if (pass == 1) break;
+      for (int i = t; i < nb; i += BLOCK) {
+        if (consts[i].flags & BC_STATIC) continue;
+        BodyState st = states[i];
+        integratePosition(st, ctx.h);
+        states[i] = st;
+      }
+      __syncthreads();
+    }
+  }
+  if (restitution) {
+    for (int a = 0; a < stageCount; ++a) {
+      const int4 st = sh.stages[a];
+      if (st.y == 0) continue;
+      F2D_UNROLL
+      for (int j = 0; j < kResidentLanes; ++j) {
+        const int lane = j * BLOCK + t;
+        if ((unsigned)(lane - st.x) < (unsigned)st.y) {
+          const float4 g = w.cons.group(0, lane);
+          if (g.x != 0.0f) {
+            const float relVel[2] = {g.y, g.z};
+            BodyState bA, bB;
+            ContactMass k;
+            loadBodies(j, bA, bB, k);
+            restitutionCore(cl[j], k, bA, bB, g.x, relVel, ctx.restitutionThreshold);
+            storeBodies(j, bA, bB);
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
+  F2D_UNROLL
+  for (int j = 0; j < kResidentLanes; ++j) {
+    const int lane = j * BLOCK + t;
+    if (lane < lanes) {
+      const float4 g = w.cons.group(0, lane);
+      const float relVel[2] = {g.y, g.z};
+      storeLane(cl[j], relVel, w.contacts[__float_as_int(g.w)]);
+    }
+  }
+}
+
+// Prepare of one contact lane in memory (any world).
+__device__ __forceinline__ void prepareWorldLane(const WorldPtrs& w, int lane, int slot, const BodyState* states,
+                                                 const SolveCtx& ctx) {
+  const Contact& c = w.contacts[slot];
+  const BodySim& sa = w.sims[c.bodyA];
+  const BodySim& sb = w.sims[c.bodyB];
+  const bool staticA = sa.type == kStatic, staticB = sb.type == kStatic;
+  ContactMass k = {sa.invMass, sa.invI, sb.invMass, sb.invI};
+  if (staticA) k.mA = 0.0f, k.iA = 0.0f;
+  if (staticB) k.mB = 0.0f, k.iB = 0.0f;
+  prepareMemoryLane(w.cons, lane, c, slot, staticA ? -1 : c.bodyA, staticB ? -1 : c.bodyB, k, states,
+                    ctx.warmStartScale);
+}
+
+// The solver stages of any world, contact lanes and joints in HBM (L2). kLds: body states
+// in LDS and the per-step body terms at `consts` in HBM; else both come from the body
+// records.
 template <int BLOCK, bool kLds>
-__device__ void solveAndFinalize(const WorldPtrs& w, SharedState& sh, BodyState* ldsStates, const SolveCtx& ctx,
-                                 int phases, int ldsBytes) {
+__device__ __forceinline__ void solveStreamed(const WorldPtrs& w, SharedState& sh, BodyState* states,
+                                              BodyConst* consts, const int* jointLanes, const SolveCtx& ctx) {
+  const WorldHeader* h = w.hdr;
+  const int nb = h->bodyCount;
+  const Cons cons = w.cons;
+  Joint* jts = w.joints;
+  const int totalLanes = sh.colorStart[kGraphColorCount];
+  const int overflowStart = sh.colorStart[kOverflowIndex];
+  const int overflowCount = sh.colorCount[kOverflowIndex];
+  const int overflowJoints = sh.jointColorCount[kOverflowIndex];
+  const int* overflowJointList = jointLanes + sh.jointColorStart[kOverflowIndex];
+  // the overflow stages (one lane, then a barrier) only when there is overflow
+  const bool anyOverflow = overflowJoints + overflowCount > 0;
+  const int stageCount = sh.stageCount;
+
+  // -- prepare joints (all), S/solver.c:967-987 -> S/joint.c:1348-1402
+  for (int i = threadIdx.x; i < h->jointCount; i += BLOCK) {
+    if (jts[i].color >= 0) prepareJoint(jts[i], w.sims, ctx.h, ctx.inv_h, ctx.warmStartScale);
+  }
+  // -- prepare contacts (all lanes), S/contact_solver.c:1438-1669
+  for (int lane = threadIdx.x; lane < totalLanes; lane += BLOCK)
+    prepareWorldLane(w, lane, lane < overflowStart ? colorLaneSlot(w, sh, lane) : w.overflow[lane - overflowStart],
+                     states, ctx);
+  __syncthreads();
+
+  for (int sub = 0; sub < ctx.subSteps; ++sub) {
+    // integrate velocities
+    for (int i = threadIdx.x; i < nb; i += BLOCK) {
+      if (kLds) {
+        BodyConst k = consts[i];
+        if (k.flags & BC_STATIC) continue;
+        BodyState st = states[i];
+        integrateVelocityConst(k, st, ctx.maxLinearSpeed, ctx.maxAngularSpeed);
+        states[i] = st;
+        if (k.flags & BC_CAPPED) w.sims[i].flags |= BF_CAPPED_STEP;
+      } else {
+        BodySim& sim = w.sims[i];
+        if (sim.setIndex != kAwakeSet) continue;
+        BodyState st = states[i];
+        integrateVelocity(sim, st, ctx.gravity, ctx.h, ctx.maxLinearSpeed, ctx.maxAngularSpeed);
+        states[i] = st;
+      }
+    }
+    __syncthreads();
+    // warm start: overflow joints, overflow contacts, then colours
+    if (anyOverflow) {
+      if (threadIdx.x == 0) {
+        for (int k = 0; k < overflowJoints; ++k)
+          if (overflowJointList[k] >= 0) warmStartJoint(jts[overflowJointList[k]], states);
+        for (int k = 0; k < overflowCount; ++k) overflowWarmStart(cons, overflowStart + k, states);
+      }
+      __syncthreads();
+    }
+    for (int a = 0; a < stageCount; ++a) {
+      const int4 st = sh.stages[a];
+      for (int k = threadIdx.x; k < st.w; k += BLOCK) warmStartJoint(jts[jointLanes[st.z + k]], states);
+      for (int k = threadIdx.x; k < st.y; k += BLOCK) warmStartMemoryLane(cons, st.x + k, states);
+      __syncthreads();
+    }
+    for (int pass = 0; pass < 2; ++pass) {
+      // solve, integrate positions, relax
+      const bool useBias = pass == 0;
+      if (anyOverflow) {
+        if (threadIdx.x == 0) {
+          for (int k = 0; k < overflowJoints; ++k)
+            if (overflowJointList[k] >= 0) solveJoint(jts[overflowJointList[k]], states, ctx.h, ctx.inv_h, useBias);
+          for (int k = 0; k < overflowCount; ++k)
+            overflowSolve(cons, overflowStart + k, states, ctx.inv_h, ctx.maxContactPushSpeed, useBias,
+                          ctx.contactSoftness, ctx.staticSoftness);
+        }
+        __syncthreads();
+      }
+      for (int a = 0; a < stageCount; ++a) {
+        const int4 st = sh.stages[a];
+        for (int k = threadIdx.x; k < st.w; k += BLOCK)
+          solveJoint(jts[jointLanes[st.z + k]], states, ctx.h, ctx.inv_h, useBias);
+        for (int k = threadIdx.x; k < st.y; k += BLOCK)
+          solveMemoryLane(cons, st.x + k, states, ctx.inv_h, -ctx.contactSpeed, useBias, ctx.contactSoftness,
+                          ctx.staticSoftness);
+        __syncthreads();
+      }
+      if (pass == 1) break;
+      for (int i = threadIdx.x; i < nb; i += BLOCK) {
+        if (kLds ? (consts[i].flags & BC_STATIC) != 0 : w.sims[i].setIndex != kAwakeSet) continue;
+        BodyState st = states[i];
+        integratePosition(st, ctx.h);
+        states[i] = st;
+      }
+      __syncthreads();
+    }
+  }
+  // restitution: overflow then colours
+  if (overflowCount > 0) {
+    if (threadIdx.x == 0) {
+      for (int k = 0; k < overflowCount; ++k)
+        overflowRestitution(cons, overflowStart + k, states, ctx.restitutionThreshold);
+    }
+    __syncthreads();
+  }
+  for (int a = 0; a < stageCount; ++a) {
+    const int4 st = sh.stages[a];
+    if (st.y == 0) continue;
+    for (int k = threadIdx.x; k < st.y; k += BLOCK)
+      restitutionMemoryLane(cons, st.x + k, states, ctx.restitutionThreshold);
+    __syncthreads();
+  }
+  // store impulses
+  for (int lane = threadIdx.x; lane < totalLanes; lane += BLOCK) {
+    Contact& c = w.contacts[cons.geti(CN_SLOT, lane)];
+    if (lane >= overflowStart) {
+      overflowStore(cons, lane, c);
+    } else {
+      storeMemoryLane(cons, lane, c);
+    }
+  }
+}
+
+// b2FinalizeBodiesTask, S/solver.c:543-726, one body per lane: transforms, AABBs, fat-AABB
+// enlargement, sleep timers, the fast bodies and the next move array.
+template <int BLOCK>
+__device__ __forceinline__ void finalizeBodies(const WorldPtrs& w, SharedState& sh, BodyState* states,
+                                               const SolveCtx& ctx) {
   WorldHeader* h = w.hdr;
   const int nb = h->bodyCount;
-  const int nc = h->contactCount;
-  BodyState* states = kLds ? ldsStates : w.states;
-  BodyConst* ldsConsts = reinterpret_cast<BodyConst*>(ldsStates + nb);  // LDS only
-  // the constraint SoA: the world's lanes in LDS behind the body terms when they fit
-  // the workgroup's LDS, else the world's region of the batch array in HBM; the
-  // same for the joints
-  Cons cons = w.cons;
-  Joint* jts = w.joints;
-  // joint ids by colour (behind the colour table of the stage launches in a split solve)
-  int* jointLanes = (phases & PH_SOLVE_PREP) ? w.scratch + kWideTableInts : w.scratch;
-
-  // b2Solve, S/solver.c:1190-1220 and :1479-1706: merge islands linked since the last
-  // step, stop when no body is awake, split the last step's candidate island
-  if (phases & PH_SOLVE) {
-    // b2MergeAwakeIslands (S/island.c:547-590). Its first loop leaves every awake
-    // island pointing at its root; here every lane walks its islands' parent chains
-    // read-only (a chain read while other lanes shorten it still ends at the same
-    // root) and writes its own island's root, then one lane merges in reverse
-    // awake order.
-    const bool merge = h->mergePending != 0;
-    if (merge) {
-      IslandCtx ic = w.isl;
-      for (int i = threadIdx.x; i < h->awakeIslandCount; i += BLOCK) {
-        const int id = ic.awakeIslands[i];
-        int root = id;
-        for (int guard = h->islandCount; ic.islands[root].parent != -1 && guard > 0; --guard)
-          root = ic.islands[root].parent;
-        if (root != id) ic.islands[id].parent = root;
-      }
-      __syncthreads();
-      // the relabelling of b2MergeIsland on all lanes: whatever belongs to an awake
-      // island with a parent (a child to merge) takes the parent's (its root's) id
-      const int ni = h->islandCap;
-      for (int i = threadIdx.x; i < nb; i += BLOCK) {
-        const int id = w.sims[i].islandId;
-        if (id < 0 || id >= ni) continue;
-        const Island& is = ic.islands[id];
-        if (is.parent != -1 && is.setIndex == kAwakeSet) w.sims[i].islandId = is.parent;
-      }
-      for (int k = threadIdx.x; k < nc; k += BLOCK) {
-        const int id = w.links[k].x;
-        if (id < 0 || id >= ni) continue;
-        const Island& is = ic.islands[id];
-        if (is.parent != -1 && is.setIndex == kAwakeSet) w.links[k].x = is.parent;
-      }
-      for (int j = threadIdx.x; j < h->jointCount; j += BLOCK) {
-        const int id = w.joints[j].islandId;
-        if (id < 0 || id >= ni) continue;
-        const Island& is = ic.islands[id];
-        if (is.parent != -1 && is.setIndex == kAwakeSet) w.joints[j].islandId = is.parent;
-      }
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-      IslandCtx ic = w.isl;
-      if (merge) mergeAwakeChildren(ic);
-      sh.noAwake = h->awakeBodyCount == 0 ? 1 : 0;
-      if (!sh.noAwake && h->splitIslandId != -1) splitIsland(ic, h->splitIslandId);
-      if (!sh.noAwake) h->splitIslandId = -1;
-    }
-    __syncthreads();
-    if (sh.noAwake) return;
-  } else if (phases & PH_FINALIZE) {
-    if (threadIdx.x == 0) sh.noAwake = h->awakeBodyCount == 0 ? 1 : 0;
-    __syncthreads();
-    if (sh.noAwake) return;
+  const IslandCtx& ic = w.isl;
+  if (threadIdx.x == 0) {
+    sh.fastCount = 0;
+    h->splitKey = 0ull;
+    h->moveBodyCount = h->awakeBodyCount;
   }
+  for (int k = threadIdx.x; k < (h->awakeIslandCount + 31) / 32; k += BLOCK) ic.awakeBits[k] = 0u;
+  // the awake order of this finalize (body move events follow it)
+  for (int k = threadIdx.x; k < h->awakeBodyCount; k += BLOCK) ic.moveOrder[k] = ic.awakeBodies[k];
+  __syncthreads();
+  int* fastList = w.scratch;  // fast bodies for the continuous-collision launch
+  for (int i = threadIdx.x; i < nb; i += BLOCK) {
+    BodySim& sim = w.sims[i];
+    if (sim.setIndex != kAwakeSet) continue;
+    BodyState st = states[i];
+    Vec2 v = st.v;
+    float wv = st.w;
+    sim.center = add(sim.center, st.dp);
+    sim.xf.q = normalizeRot(mulRot(st.dq, sim.xf.q));
+    float maxVelocity = length(v) + absf(wv) * sim.maxExtent;
+    float maxDeltaPosition = length(st.dp) + absf(st.dq.s) * sim.maxExtent;
+    float positionSleepFactor = 0.5f;
+    float sleepVelocity = maxf(maxVelocity, positionSleepFactor * ctx.inv_dt * maxDeltaPosition);
+    st.dp = {0.0f, 0.0f};
+    st.dq = {1.0f, 0.0f};
+    sim.xf.p = sub(sim.center, rotate(sim.xf.q, sim.localCenter));
+    sim.force = {0.0f, 0.0f};
+    sim.torque = 0.0f;
+    // isSpeedCapped reports this step's capping (body->isSpeedCapped = sim->isSpeedCapped)
+    bool capped = (sim.flags & BF_CAPPED_STEP) != 0;
+    int flags = sim.flags & ~(BF_IS_FAST | BF_ENLARGED | BF_SPEED_CAPPED | BF_CAPPED_STEP | BF_FELL_ASLEEP);
+    if (capped) flags |= BF_SPEED_CAPPED;
+    bool isFast = false;
+    if (!ctx.enableSleep || (sim.flags & BF_ENABLE_SLEEP) == 0 || sleepVelocity > sim.sleepThreshold) {
+      sim.sleepTime = 0.0f;
+      if (sim.type == kDynamic && ctx.enableContinuous && maxVelocity * ctx.dt > 0.5f * sim.minExtent) {
+        // the continuous-collision launch sweeps this body (b2SolveContinuous)
+        isFast = true;
+        int slot = atomicAdd(&sh.fastCount, 1);
+        fastList[slot] = i;
+      } else {
+        sim.center0 = sim.center;
+        sim.rotation0 = sim.xf.q;
+      }
+    } else {
+      sim.center0 = sim.center;
+      sim.rotation0 = sim.xf.q;
+      sim.sleepTime += ctx.dt;
+    }
+    // any body of an island keeps it awake; the sleepiest body (first in the awake
+    // order on ties) of an island with removed constraints names the island to
+    // split next step (S/solver.c:658-676)
+    if (ctx.enableSleep && sim.islandId >= 0 && sim.islandId < h->islandCap) {
+      const Island& is = ic.islands[sim.islandId];
+      if (sim.sleepTime < kTimeToSleep) {
+        atomicOr(&ic.awakeBits[is.localIndex >> 5], 1u << (is.localIndex & 31));
+      } else if (is.removeCount > 0) {
+        unsigned long long key = ((unsigned long long)__float_as_uint(sim.sleepTime) << 32) |
+                                 (unsigned long long)(0xFFFFFFFFu - (uint32_t)sim.localIndex);
+        atomicMax(&h->splitKey, key);
+      }
+    }
+    Xf xf = sim.xf;
+    int rank = 0;
+    bool enlargedBody = false;
+    const bool bullet = (sim.flags & BF_BULLET) != 0;
+    for (int s = sim.headShape; s >= 0 && rank < h->shapeCount; s = w.shapes[s].next, ++rank) {
+      Shape& shape = w.shapes[s];
+      if (isFast) {
+        // fast shapes get their AABBs from the continuous sweep; a fast bullet
+        // joins the move buffer with every shape (S/solver.c:1866-1879)
+        if (bullet) {
+          shape.flags |= SF_MOVED;
+          shape.moveRank = (sim.localIndex << 8) | (rank < 255 ? rank : 255);
+          enlargedBody = true;
+        }
+        continue;
+      }
+      AABB aabb = computeShapeAABB(w.geoms[s], xf);
+      aabb.lo.x -= kSpeculativeDistance;
+      aabb.lo.y -= kSpeculativeDistance;
+      aabb.hi.x += kSpeculativeDistance;
+      aabb.hi.y += kSpeculativeDistance;
+      shape.aabb = aabb;
+      if (!aabbContains(shape.fat, aabb)) {
+        AABB fat;
+        fat.lo.x = aabb.lo.x - kAabbMargin;
+        fat.lo.y = aabb.lo.y - kAabbMargin;
+        fat.hi.x = aabb.hi.x + kAabbMargin;
+        fat.hi.y = aabb.hi.y + kAabbMargin;
+        shape.fat = fat;
+        shape.flags |= SF_TREE_PENDING;
+        // enlarged proxy joins the move buffer in sim order (S/solver.c:1848-1903)
+        shape.flags |= SF_MOVED;
+        shape.moveRank = (sim.localIndex << 8) | (rank < 255 ? rank : 255);
+        enlargedBody = true;
+      }
+    }
+    if (enlargedBody) flags |= BF_ENLARGED;
+    if (isFast) flags |= BF_IS_FAST;
+    sim.flags = flags;
+    w.states[i] = st;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    h->fastCount = sh.fastCount;
+    h->sleepPending = ctx.enableSleep ? 1 : 0;
+  }
+}
 
+// The solve and finalize phases of one world. LDS holds, as far as ldsBytes go, the body
+// states and per-step body terms (64 B a body, one slot more for the static bodies) and
+// the joints: then the contacts stay in registers (solveResident) unless there are too
+// many, or overflow constraints, or joints of other types (out-of-line calls). Otherwise
+// the states alone (32 B a body), otherwise nothing; contacts and joints then stream from
+// L2 (solveStreamed).
+template <int BLOCK>
+__device__ __forceinline__ void solveAndFinalize(const WorldPtrs& w, SharedState& sh, char* lds, const SolveCtx& ctx,
+                                                 int phases, int ldsBytes) {
+  WorldHeader* h = w.hdr;
+  const int nb = h->bodyCount;
+  BodyState* ldsStates = reinterpret_cast<BodyState*>(lds);
+  const bool inLds = (long)nb * (long)sizeof(BodyState) <= ldsBytes;
   if (phases & PH_SOLVE) {
-    // -- bucket touching constraints by colour (overflow keeps its list order)
-    if (threadIdx.x < kGraphColorCount) {
-      sh.colorCount[threadIdx.x] = 0;
-      sh.colorFill[threadIdx.x] = 0;
-      sh.jointColorCount[threadIdx.x] = 0;
-      sh.jointColorFill[threadIdx.x] = 0;
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < nc; i += BLOCK) {
-      int color = w.ccolor[i];
-      if (color >= 0 && color < kOverflowIndex) atomicAdd(&sh.colorCount[color], 1);
-    }
-    for (int i = threadIdx.x; i < h->jointCount; i += BLOCK) {
-      const Joint& j = w.joints[i];
-      if (j.color >= 0) atomicAdd(&sh.jointColorCount[j.color], 1);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int s = 0, sj = 0, active = 0;
-      for (int k = 0; k < kOverflowIndex; ++k) {
-        sh.colorStart[k] = s;
-        s += sh.colorCount[k];
-        sh.jointColorStart[k] = sj;
-        sj += sh.jointColorCount[k];
-        active += (sh.colorCount[k] + sh.jointColorCount[k]) > 0 ? 1 : 0;
-      }
-      sh.colorStart[kOverflowIndex] = s;
-      sh.colorCount[kOverflowIndex] = h->overflowCount;
-      sh.colorStart[kGraphColorCount] = s + h->overflowCount;
-      sh.jointColorStart[kOverflowIndex] = sj;
-      h->activeColors = active;
-    }
-    __syncthreads();
-    // LDS behind the body terms: the joints (copied in here, back after the
-    // substeps), then the constraint lanes, as far as each fits
-    if (kLds) {
-      const long lanes = sh.colorStart[kGraphColorCount];
-      long off = (long)nb * (long)(sizeof(BodyState) + sizeof(BodyConst));
-      const long jointBytes = (long)h->jointCount * (long)sizeof(Joint);
-      if (h->jointCount > 0 && off + jointBytes <= ldsBytes) {
-        jts = reinterpret_cast<Joint*>(reinterpret_cast<char*>(ldsStates) + off);
-        off += jointBytes;
-      }
-      if (lanes > 0 && off + 4L * CN_FIELD_COUNT * lanes <= ldsBytes) {
-        cons.f = reinterpret_cast<float*>(reinterpret_cast<char*>(ldsStates) + off);
-        cons.stride = lanes;
-        off += 4L * CN_FIELD_COUNT * lanes;
-      }
-      // the joint ids by colour, read at every colour stage
-      if (h->jointCount > 0 && off + 4L * h->jointCount <= ldsBytes) {
-        jointLanes = reinterpret_cast<int*>(reinterpret_cast<char*>(ldsStates) + off);
-      }
-    }
-    for (int i = threadIdx.x; i < nc; i += BLOCK) {
-      int color = w.ccolor[i];
-      if (color >= 0 && color < kOverflowIndex) {
-        int lane = sh.colorStart[color] + atomicAdd(&sh.colorFill[color], 1);
-        cons.seti(CN_SLOT, lane, i);
-      }
-    }
-    for (int i = threadIdx.x; i < h->overflowCount; i += BLOCK) {
-      cons.seti(CN_SLOT, sh.colorStart[kOverflowIndex] + i, w.overflow[i]);
-    }
-    for (int i = threadIdx.x; i < h->jointCount; i += BLOCK) {
-      const Joint& j = w.joints[i];
-      if (j.color >= 0 && j.color < kOverflowIndex) {
-        jointLanes[sh.jointColorStart[j.color] + atomicAdd(&sh.jointColorFill[j.color], 1)] = i;
-      }
-    }
-    if (threadIdx.x == 0 && sh.jointColorCount[kOverflowIndex] > 0) {
-      // overflow joints are solved one after another in their colour's array order
-      int* list = jointLanes + sh.jointColorStart[kOverflowIndex];
-      const int n = sh.jointColorCount[kOverflowIndex];
-      for (int k = 0; k < n; ++k) list[k] = -1;
-      for (int i = 0; i < h->jointCount; ++i) {
-        const Joint& j = w.joints[i];
-        if (j.color == kOverflowIndex && j.localIndex >= 0 && j.localIndex < n) list[j.localIndex] = i;
-      }
-      for (int k = 0; k < n; ++k)
-        if (list[k] < 0) h->error |= ERR_OVERFLOW_CAP;
-    }
-    // body states and per-step body terms into LDS
-    if (kLds) {
-      for (int i = threadIdx.x; i < nb; i += BLOCK) {
-        ldsStates[i] = w.states[i];
-        ldsConsts[i] = makeBodyConst(w.sims[i], ctx.gravity, ctx.h);
-      }
-      if (jts != w.joints) {
-        const int words = h->jointCount * (int)(sizeof(Joint) / sizeof(float4));
-        const float4* src = reinterpret_cast<const float4*>(w.joints);
-        float4* dst = reinterpret_cast<float4*>(jts);
-        for (int i = threadIdx.x; i < words; i += BLOCK) dst[i] = src[i];
-      }
-    }
-    __syncthreads();
+    if (!solveIslands<BLOCK>(w, sh)) return;
+    solveColors<BLOCK>(w, sh);
+    const int lanes = sh.colorStart[kGraphColorCount];
     if (phases & PH_SOLVE_PREP) {
-      // the colour table of the stage launches (wideStageKernel)
+      // the joint ids by colour, the contact slots and the colour table of the stage
+      // launches (wideStageKernel)
+      listJoints<BLOCK>(w, sh, w.scratch + kWideTableInts);
+      const int overflowStart = sh.colorStart[kOverflowIndex];
+      for (int lane = threadIdx.x; lane < lanes; lane += BLOCK)
+        w.cons.seti(CN_SLOT, lane, lane < overflowStart ? colorLaneSlot(w, sh, lane) : w.overflow[lane - overflowStart]);
       int* table = w.scratch;
       if (threadIdx.x < kGraphColorCount) {
         table[kWideColorCount + threadIdx.x] = sh.colorCount[threadIdx.x];
@@ -1407,286 +1799,67 @@ __device__ void solveAndFinalize(const WorldPtrs& w, SharedState& sh, BodyState*
       if (threadIdx.x <= kGraphColorCount) table[kWideColorStart + threadIdx.x] = sh.colorStart[threadIdx.x];
       return;
     }
-    const int totalLanes = sh.colorStart[kGraphColorCount];
-    const int overflowStart = sh.colorStart[kOverflowIndex];
-    const int overflowCount = sh.colorCount[kOverflowIndex];
-    const int coloredJoints = sh.jointColorStart[kOverflowIndex];
-    const int overflowJoints = sh.jointColorCount[kOverflowIndex];
-    const int* overflowJointList = jointLanes + coloredJoints;
-    // the overflow stages (one lane, then a barrier) only when there is overflow
-    const bool anyOverflow = overflowJoints + overflowCount > 0;
-
-    // -- prepare joints (all), S/solver.c:967-987 -> S/joint.c:1348-1402
-    for (int i = threadIdx.x; i < h->jointCount; i += BLOCK) {
-      if (jts[i].color >= 0) prepareJoint(jts[i], w.sims, ctx.h, ctx.inv_h, ctx.warmStartScale);
-    }
-    // -- prepare contacts (all lanes), S/contact_solver.c:1438-1669
-    for (int lane = threadIdx.x; lane < totalLanes; lane += BLOCK) {
-      int slot = cons.geti(CN_SLOT, lane);
-      const Contact& c = w.contacts[slot];
-      bool staticA, staticB;
-      float mA, iA, mB, iB;
-      if (kLds) {
-        const BodyConst& ka = ldsConsts[c.bodyA];
-        const BodyConst& kb = ldsConsts[c.bodyB];
-        staticA = (ka.flags & BC_STATIC) != 0;
-        staticB = (kb.flags & BC_STATIC) != 0;
-        mA = ka.invMass, iA = ka.invI, mB = kb.invMass, iB = kb.invI;
-      } else {
-        const BodySim& sa = w.sims[c.bodyA];
-        const BodySim& sb = w.sims[c.bodyB];
-        staticA = sa.type == kStatic;
-        staticB = sb.type == kStatic;
-        mA = sa.invMass, iA = sa.invI, mB = sb.invMass, iB = sb.invI;
-      }
-      int ia = staticA ? -1 : c.bodyA;
-      int ib = staticB ? -1 : c.bodyB;
-      if (staticA) mA = 0.0f, iA = 0.0f;
-      if (staticB) mB = 0.0f, iB = 0.0f;
-      prepareContactLane(cons, lane, c, slot, ia, ib, mA, iA, mB, iB, states, ctx.contactSoftness,
-                         ctx.staticSoftness, ctx.warmStartScale);
-    }
-    __syncthreads();
-
-    for (int sub = 0; sub < ctx.subSteps; ++sub) {
-      // integrate velocities
-      for (int i = threadIdx.x; i < nb; i += BLOCK) {
-        if (kLds) {
-          BodyConst k = ldsConsts[i];
-          if (k.flags & BC_STATIC) continue;
-          BodyState st = states[i];
-          integrateVelocityConst(k, st, ctx.maxLinearSpeed, ctx.maxAngularSpeed);
-          states[i] = st;
-          ldsConsts[i].flags = k.flags;
+    const int nj = h->jointCount;
+    const long bodyBytes = (long)(nb + 1) * (long)(sizeof(BodyState) + sizeof(BodyConst));
+    const long jointBytes = (long)nj * (long)(sizeof(Joint) + sizeof(int));
+    const bool resident = bodyBytes + jointBytes <= ldsBytes && nb < 0xFFFF && sh.otherJoints == 0 &&
+                          sh.colorCount[kOverflowIndex] == 0 && sh.jointColorCount[kOverflowIndex] == 0 &&
+                          lanes <= kResidentLanes * BLOCK;
+    if (resident) {
+      BodyConst* consts = reinterpret_cast<BodyConst*>(ldsStates + nb + 1);
+      Joint* jts = reinterpret_cast<Joint*>(consts + nb + 1);
+      int* jointLanes = reinterpret_cast<int*>(jts + nj);
+      listJoints<BLOCK>(w, sh, jointLanes);
+      for (int i = threadIdx.x; i <= nb; i += BLOCK) {
+        if (i < nb) {
+          ldsStates[i] = w.states[i];
+          consts[i] = makeBodyConst(w.sims[i], ctx.gravity, ctx.h);
         } else {
-          BodySim& sim = w.sims[i];
-          if (sim.setIndex != kAwakeSet) continue;
-          BodyState st = states[i];
-          integrateVelocity(sim, st, ctx.gravity, ctx.h, ctx.maxLinearSpeed, ctx.maxAngularSpeed);
-          states[i] = st;
+          ldsStates[i] = identityState();
+          BodyConst none = {};
+          none.flags = BC_STATIC;
+          consts[i] = none;
         }
       }
+      const int words = nj * (int)(sizeof(Joint) / sizeof(float4));
+      for (int i = threadIdx.x; i < words; i += BLOCK)
+        reinterpret_cast<float4*>(jts)[i] = reinterpret_cast<const float4*>(w.joints)[i];
       __syncthreads();
-      // warm start: overflow joints, overflow contacts, then colours
-      if (anyOverflow) {
-        if (threadIdx.x == 0) {
-          for (int k = 0; k < overflowJoints; ++k)
-            if (overflowJointList[k] >= 0) warmStartJoint(jts[overflowJointList[k]], states);
-          for (int k = 0; k < overflowCount; ++k) overflowWarmStart(cons, overflowStart + k, states);
+      solveResident<BLOCK>(w, sh, ldsStates, consts, jts, jointLanes, ctx);
+      // the joints' impulses and prepared data back to HBM
+      for (int i = threadIdx.x; i < words; i += BLOCK)
+        reinterpret_cast<float4*>(w.joints)[i] = reinterpret_cast<const float4*>(jts)[i];
+    } else {
+      // scratch: joint ids by colour, then (behind what finalize's fast list may take) the
+      // per-step body terms
+      listJoints<BLOCK>(w, sh, w.scratch);
+      const long at = ((long)nj + nb + 3) & ~3L;
+      const bool terms = inLds && at + (long)nb * (long)(sizeof(BodyConst) / 4) <= h->scratchCap;
+      if (terms) {
+        BodyConst* consts = reinterpret_cast<BodyConst*>(w.scratch + at);
+        for (int i = threadIdx.x; i < nb; i += BLOCK) {
+          ldsStates[i] = w.states[i];
+          consts[i] = makeBodyConst(w.sims[i], ctx.gravity, ctx.h);
         }
         __syncthreads();
-      }
-      for (int col = 0; col < kOverflowIndex; ++col) {
-        int cnt = sh.colorCount[col], jcnt = sh.jointColorCount[col];
-        if (cnt + jcnt == 0) continue;
-        for (int k = threadIdx.x; k < jcnt; k += BLOCK)
-          warmStartJoint(jts[jointLanes[sh.jointColorStart[col] + k]], states);
-        for (int k = threadIdx.x; k < cnt; k += BLOCK) warmStartLane(cons, sh.colorStart[col] + k, states);
-        __syncthreads();
-      }
-      // solve
-      if (anyOverflow) {
-        if (threadIdx.x == 0) {
-          for (int k = 0; k < overflowJoints; ++k)
-            if (overflowJointList[k] >= 0)
-              solveJoint(jts[overflowJointList[k]], states, ctx.h, ctx.inv_h, true);
-          for (int k = 0; k < overflowCount; ++k)
-            overflowSolve(cons, overflowStart + k, states, ctx.inv_h, ctx.maxContactPushSpeed, true);
-        }
-        __syncthreads();
-      }
-      for (int col = 0; col < kOverflowIndex; ++col) {
-        int cnt = sh.colorCount[col], jcnt = sh.jointColorCount[col];
-        if (cnt + jcnt == 0) continue;
-        for (int k = threadIdx.x; k < jcnt; k += BLOCK)
-          solveJoint(jts[jointLanes[sh.jointColorStart[col] + k]], states, ctx.h, ctx.inv_h, true);
-        for (int k = threadIdx.x; k < cnt; k += BLOCK)
-          solveLane(cons, sh.colorStart[col] + k, states, ctx.inv_h, -ctx.contactSpeed, true);
-        __syncthreads();
-      }
-      // integrate positions
-      for (int i = threadIdx.x; i < nb; i += BLOCK) {
-        if (kLds ? (ldsConsts[i].flags & BC_STATIC) != 0 : w.sims[i].setIndex != kAwakeSet) continue;
-        BodyState st = states[i];
-        integratePosition(st, ctx.h);
-        states[i] = st;
-      }
-      __syncthreads();
-      // relax
-      if (anyOverflow) {
-        if (threadIdx.x == 0) {
-          for (int k = 0; k < overflowJoints; ++k)
-            if (overflowJointList[k] >= 0)
-              solveJoint(jts[overflowJointList[k]], states, ctx.h, ctx.inv_h, false);
-          for (int k = 0; k < overflowCount; ++k)
-            overflowSolve(cons, overflowStart + k, states, ctx.inv_h, ctx.maxContactPushSpeed, false);
-        }
-        __syncthreads();
-      }
-      for (int col = 0; col < kOverflowIndex; ++col) {
-        int cnt = sh.colorCount[col], jcnt = sh.jointColorCount[col];
-        if (cnt + jcnt == 0) continue;
-        for (int k = threadIdx.x; k < jcnt; k += BLOCK)
-          solveJoint(jts[jointLanes[sh.jointColorStart[col] + k]], states, ctx.h, ctx.inv_h, false);
-        for (int k = threadIdx.x; k < cnt; k += BLOCK)
-          solveLane(cons, sh.colorStart[col] + k, states, ctx.inv_h, -ctx.contactSpeed, false);
-        __syncthreads();
-      }
-    }
-    // the joints' impulses and prepared data back to HBM
-    if (jts != w.joints) {
-      const int words = h->jointCount * (int)(sizeof(Joint) / sizeof(float4));
-      const float4* src = reinterpret_cast<const float4*>(jts);
-      float4* dst = reinterpret_cast<float4*>(w.joints);
-      for (int i = threadIdx.x; i < words; i += BLOCK) dst[i] = src[i];
-    }
-    // restitution: overflow then colours
-    if (overflowCount > 0) {
-      if (threadIdx.x == 0) {
-        for (int k = 0; k < overflowCount; ++k)
-          overflowRestitution(cons, overflowStart + k, states, ctx.restitutionThreshold);
-      }
-      __syncthreads();
-    }
-    for (int col = 0; col < kOverflowIndex; ++col) {
-      int cnt = sh.colorCount[col];
-      if (cnt == 0) continue;
-      for (int k = threadIdx.x; k < cnt; k += BLOCK)
-        restitutionLane(cons, sh.colorStart[col] + k, states, ctx.restitutionThreshold);
-      __syncthreads();
-    }
-    // store impulses
-    for (int lane = threadIdx.x; lane < totalLanes; lane += BLOCK) {
-      int slot = cons.geti(CN_SLOT, lane);
-      if (lane >= overflowStart) {
-        overflowStore(cons, lane, w.contacts[slot]);
+        solveStreamed<BLOCK, true>(w, sh, ldsStates, consts, w.scratch, ctx);
       } else {
-        storeLane(cons, lane, w.contacts[slot]);
+        __syncthreads();
+        solveStreamed<BLOCK, false>(w, sh, w.states, nullptr, w.scratch, ctx);
+        __syncthreads();
+        if (phases & PH_FINALIZE) finalizeBodies<BLOCK>(w, sh, w.states, ctx);
+        return;
       }
     }
-    (void)coloredJoints;
     __syncthreads();
-  } else if (kLds) {
-    for (int i = threadIdx.x; i < nb; i += BLOCK) ldsStates[i] = w.states[i];
-    __syncthreads();
-  }
-
-  if (phases & PH_FINALIZE) {
-    // b2FinalizeBodiesTask, S/solver.c:543-726
-    const IslandCtx& ic = w.isl;
-    if (threadIdx.x == 0) {
-      sh.fastCount = 0;
-      h->splitKey = 0ull;
-      h->moveBodyCount = h->awakeBodyCount;
+    if (phases & PH_FINALIZE) {
+      finalizeBodies<BLOCK>(w, sh, ldsStates, ctx);
+    } else {
+      for (int i = threadIdx.x; i < nb; i += BLOCK) w.states[i] = ldsStates[i];
     }
-    for (int k = threadIdx.x; k < (h->awakeIslandCount + 31) / 32; k += BLOCK) ic.awakeBits[k] = 0u;
-    // the awake order of this finalize (body move events follow it)
-    for (int k = threadIdx.x; k < h->awakeBodyCount; k += BLOCK) ic.moveOrder[k] = ic.awakeBodies[k];
-    __syncthreads();
-    int* fastList = w.scratch;  // fast bodies for the continuous-collision launch
-    for (int i = threadIdx.x; i < nb; i += BLOCK) {
-      BodySim& sim = w.sims[i];
-      if (sim.setIndex != kAwakeSet) continue;
-      BodyState st = states[i];
-      Vec2 v = st.v;
-      float wv = st.w;
-      sim.center = add(sim.center, st.dp);
-      sim.xf.q = normalizeRot(mulRot(st.dq, sim.xf.q));
-      float maxVelocity = length(v) + absf(wv) * sim.maxExtent;
-      float maxDeltaPosition = length(st.dp) + absf(st.dq.s) * sim.maxExtent;
-      float positionSleepFactor = 0.5f;
-      float sleepVelocity = maxf(maxVelocity, positionSleepFactor * ctx.inv_dt * maxDeltaPosition);
-      st.dp = {0.0f, 0.0f};
-      st.dq = {1.0f, 0.0f};
-      sim.xf.p = sub(sim.center, rotate(sim.xf.q, sim.localCenter));
-      sim.force = {0.0f, 0.0f};
-      sim.torque = 0.0f;
-      // isSpeedCapped reports this step's capping (body->isSpeedCapped = sim->isSpeedCapped)
-      bool capped = kLds ? (ldsConsts[i].flags & BC_CAPPED) != 0 : (sim.flags & BF_CAPPED_STEP) != 0;
-      int flags = sim.flags & ~(BF_IS_FAST | BF_ENLARGED | BF_SPEED_CAPPED | BF_CAPPED_STEP | BF_FELL_ASLEEP);
-      if (capped) flags |= BF_SPEED_CAPPED;
-      bool isFast = false;
-      if (!ctx.enableSleep || (sim.flags & BF_ENABLE_SLEEP) == 0 || sleepVelocity > sim.sleepThreshold) {
-        sim.sleepTime = 0.0f;
-        if (sim.type == kDynamic && ctx.enableContinuous && maxVelocity * ctx.dt > 0.5f * sim.minExtent) {
-          // the continuous-collision launch sweeps this body (b2SolveContinuous)
-          isFast = true;
-          int slot = atomicAdd(&sh.fastCount, 1);
-          fastList[slot] = i;
-        } else {
-          sim.center0 = sim.center;
-          sim.rotation0 = sim.xf.q;
-        }
-      } else {
-        sim.center0 = sim.center;
-        sim.rotation0 = sim.xf.q;
-        sim.sleepTime += ctx.dt;
-      }
-      // any body of an island keeps it awake; the sleepiest body (first in the awake
-      // order on ties) of an island with removed constraints names the island to
-      // split next step (S/solver.c:658-676)
-      if (ctx.enableSleep && sim.islandId >= 0 && sim.islandId < h->islandCap) {
-        const Island& is = ic.islands[sim.islandId];
-        if (sim.sleepTime < kTimeToSleep) {
-          atomicOr(&ic.awakeBits[is.localIndex >> 5], 1u << (is.localIndex & 31));
-        } else if (is.removeCount > 0) {
-          unsigned long long key = ((unsigned long long)__float_as_uint(sim.sleepTime) << 32) |
-                                   (unsigned long long)(0xFFFFFFFFu - (uint32_t)sim.localIndex);
-          atomicMax(&h->splitKey, key);
-        }
-      }
-      Xf xf = sim.xf;
-      int rank = 0;
-      bool enlargedBody = false;
-      const bool bullet = (sim.flags & BF_BULLET) != 0;
-      for (int s = sim.headShape; s >= 0 && rank < h->shapeCount; s = w.shapes[s].next, ++rank) {
-        Shape& shape = w.shapes[s];
-        if (isFast) {
-          // fast shapes get their AABBs from the continuous sweep; a fast bullet
-          // joins the move buffer with every shape (S/solver.c:1866-1879)
-          if (bullet) {
-            shape.flags |= SF_MOVED;
-            shape.moveRank = (sim.localIndex << 8) | (rank < 255 ? rank : 255);
-            enlargedBody = true;
-          }
-          continue;
-        }
-        AABB aabb = computeShapeAABB(w.geoms[s], xf);
-        aabb.lo.x -= kSpeculativeDistance;
-        aabb.lo.y -= kSpeculativeDistance;
-        aabb.hi.x += kSpeculativeDistance;
-        aabb.hi.y += kSpeculativeDistance;
-        shape.aabb = aabb;
-        if (!aabbContains(shape.fat, aabb)) {
-          AABB fat;
-          fat.lo.x = aabb.lo.x - kAabbMargin;
-          fat.lo.y = aabb.lo.y - kAabbMargin;
-          fat.hi.x = aabb.hi.x + kAabbMargin;
-          fat.hi.y = aabb.hi.y + kAabbMargin;
-          shape.fat = fat;
-          shape.flags |= SF_TREE_PENDING;
-          // enlarged proxy joins the move buffer in sim order (S/solver.c:1848-1903)
-          shape.flags |= SF_MOVED;
-          shape.moveRank = (sim.localIndex << 8) | (rank < 255 ? rank : 255);
-          enlargedBody = true;
-        }
-      }
-      if (enlargedBody) flags |= BF_ENLARGED;
-      if (isFast) flags |= BF_IS_FAST;
-      sim.flags = flags;
-      w.states[i] = st;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      h->fastCount = sh.fastCount;
-      h->sleepPending = ctx.enableSleep ? 1 : 0;
-    }
-  } else if (kLds && (phases & PH_SOLVE)) {
-    for (int i = threadIdx.x; i < nb; i += BLOCK) {
-      w.states[i] = ldsStates[i];
-      if (ldsConsts[i].flags & BC_CAPPED) w.sims[i].flags |= BF_CAPPED_STEP;
-    }
-    __syncthreads();
+  } else if (phases & PH_FINALIZE) {
+    if (h->awakeBodyCount == 0) return;
+    finalizeBodies<BLOCK>(w, sh, w.states, ctx);
   }
 }
 
@@ -1784,7 +1957,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void n
 }
 
 template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void solveKernel(BatchView b, StepParams sp, const int* worldList, int ldsBytes) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void solveKernel(BatchView b, StepParams sp, const int* worldList, int ldsBytes) {
   __shared__ SharedState sh;
   extern __shared__ __align__(16) char lds[];
   const int wi = worldList ? worldList[blockIdx.x] : blockIdx.x;
@@ -1792,11 +1965,7 @@ __global__ __launch_bounds__(BLOCK) void solveKernel(BatchView b, StepParams sp,
   WorldPtrs w = worldPtrs(b, h);
   SolveCtx ctx;
   stepContext(h, sp, ctx);
-  if (h->bodyCount * (int)(sizeof(BodyState) + sizeof(BodyConst)) <= ldsBytes) {
-    solveAndFinalize<BLOCK, true>(w, sh, reinterpret_cast<BodyState*>(lds), ctx, sp.phases, ldsBytes);
-  } else {
-    solveAndFinalize<BLOCK, false>(w, sh, nullptr, ctx, sp.phases, ldsBytes);
-  }
+  solveAndFinalize<BLOCK>(w, sh, lds, ctx, sp.phases, ldsBytes);
   if (threadIdx.x == 0 && (sp.phases & PH_NO_COUNT) == 0) h->stepIndex += 1;
 }
 
@@ -1837,18 +2006,7 @@ __global__ __launch_bounds__(256) void wideStageKernel(BatchView b, StepParams s
       if (jts[i].color >= 0) prepareJoint(jts[i], w.sims, ctx.h, ctx.inv_h, ctx.warmStartScale);
     const int totalLanes = table[kWideColorStart + kGraphColorCount];
     for (int lane = gtid; lane < totalLanes; lane += stride) {
-      const int slot = cons.geti(CN_SLOT, lane);
-      const Contact& c = w.contacts[slot];
-      const BodySim& sa = w.sims[c.bodyA];
-      const BodySim& sb = w.sims[c.bodyB];
-      const bool staticA = sa.type == kStatic, staticB = sb.type == kStatic;
-      float mA = sa.invMass, iA = sa.invI, mB = sb.invMass, iB = sb.invI;
-      const int ia = staticA ? -1 : c.bodyA;
-      const int ib = staticB ? -1 : c.bodyB;
-      if (staticA) mA = 0.0f, iA = 0.0f;
-      if (staticB) mB = 0.0f, iB = 0.0f;
-      prepareContactLane(cons, lane, c, slot, ia, ib, mA, iA, mB, iB, states, ctx.contactSoftness,
-                         ctx.staticSoftness, ctx.warmStartScale);
+      prepareWorldLane(w, lane, cons.geti(CN_SLOT, lane), states, ctx);
     }
   } else if (stage == WS_INTEGRATE_VEL) {
     for (int i = gtid; i < nb; i += stride) {
@@ -1873,7 +2031,7 @@ __global__ __launch_bounds__(256) void wideStageKernel(BatchView b, StepParams s
       if (lane >= overflowStart) {
         overflowStore(cons, lane, w.contacts[slot]);
       } else {
-        storeLane(cons, lane, w.contacts[slot]);
+        storeMemoryLane(cons, lane, w.contacts[slot]);
       }
     }
   } else if (color == kOverflowIndex) {
@@ -1892,22 +2050,24 @@ __global__ __launch_bounds__(256) void wideStageKernel(BatchView b, StepParams s
       for (int k = 0; k < jcnt; ++k)
         if (jointList[k] >= 0) solveJoint(jts[jointList[k]], states, ctx.h, ctx.inv_h, useBias);
       for (int k = 0; k < cnt; ++k)
-        overflowSolve(cons, start + k, states, ctx.inv_h, ctx.maxContactPushSpeed, useBias);
+        overflowSolve(cons, start + k, states, ctx.inv_h, ctx.maxContactPushSpeed, useBias, ctx.contactSoftness,
+                      ctx.staticSoftness);
     }
   } else {
     const int start = table[kWideColorStart + color], cnt = table[kWideColorCount + color];
     const int jstart = table[kWideJointStart + color], jcnt = table[kWideJointCount + color];
     if (stage == WS_RESTITUTION) {
-      for (int k = gtid; k < cnt; k += stride) restitutionLane(cons, start + k, states, ctx.restitutionThreshold);
+      for (int k = gtid; k < cnt; k += stride) restitutionMemoryLane(cons, start + k, states, ctx.restitutionThreshold);
     } else if (stage == WS_WARM) {
       for (int k = gtid; k < jcnt; k += stride) warmStartJoint(jts[jointLanes[jstart + k]], states);
-      for (int k = gtid; k < cnt; k += stride) warmStartLane(cons, start + k, states);
+      for (int k = gtid; k < cnt; k += stride) warmStartMemoryLane(cons, start + k, states);
     } else {
       const bool useBias = stage == WS_SOLVE;
       for (int k = gtid; k < jcnt; k += stride)
         solveJoint(jts[jointLanes[jstart + k]], states, ctx.h, ctx.inv_h, useBias);
       for (int k = gtid; k < cnt; k += stride)
-        solveLane(cons, start + k, states, ctx.inv_h, -ctx.contactSpeed, useBias);
+        solveMemoryLane(cons, start + k, states, ctx.inv_h, -ctx.contactSpeed, useBias, ctx.contactSoftness,
+                        ctx.staticSoftness);
     }
   }
 }

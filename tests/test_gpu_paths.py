@@ -50,8 +50,8 @@ def container(bodies: int, seed: int, bullets: float = 0.0, sleep: bool = False,
     return spec, np.concatenate([fg[walls], fg[pick]]).tobytes()
 
 
-def follow(spec: bytes, geoms: bytes, steps: int, **batch):
-    b = F.Batch(spec, **batch)
+def follow(spec: bytes, geoms: bytes, steps: int, b: F.Batch | None = None):
+    b = b or F.Batch(spec)
     raw = b.export(0)
     prev = S.parse_one(raw)
     for k in range(1, steps + 1):
@@ -71,3 +71,17 @@ def follow(spec: bytes, geoms: bytes, steps: int, **batch):
 def test_bullets(gpu, bodies, bullets, sleep, steps):
     spec, geoms = container(bodies, 11 + bodies, bullets=bullets, sleep=sleep, speed=25.0)
     follow(spec, geoms, steps)
+
+
+# the solver stages: contacts in registers (up to three a lane), or streamed with the bodies
+# in LDS (more contacts than that, or worlds above 1,024 bodies) or with nothing in LDS;
+# lanes a power of two from 64, worlds on both sides of what they hold
+@pytest.mark.parametrize("bodies,block,steps", [(1, 64, 30), (2, 1024, 30), (63, 64, 40), (64, 64, 40), (130, 64, 60),
+                                                (130, 128, 60), (500, 64, 40), (500, 256, 40), (500, 512, 40),
+                                                (1000, 1024, 30), (1023, 512, 20), (1024, 1024, 20), (3000, 1024, 12),
+                                                (4096, 256, 6), (4097, 1024, 6)])
+def test_solver_stages(gpu, bodies, block, steps):
+    spec, geoms = container(bodies, 23 + bodies, speed=4.0)
+    b = F.Batch(spec)
+    b.set_block(block)
+    follow(spec, geoms, steps, b)
