@@ -2406,40 +2406,57 @@ __device__ __forceinline__ Vec2 boxExtents(const AABB& a) {  // b2AABB_Extents
 // it and are marked enlarged. The step's tree launch applies them at the start of
 // the next step; queries between steps walk the trees and need them now. The
 // boxes and marks do not depend on the order of the leaves, and the next tree
-// launch rebuilds the marked nodes as it would have. Thread 0 of one workgroup per
-// world walks up from each pending leaf.
-__global__ __launch_bounds__(64) void enlargePendingKernel(BatchView b) {
+// launch rebuilds the marked nodes as it would have. A workgroup per world, a pending leaf
+// per lane, each walking up on its own: a box only grows (a bound that a walk finds
+// already beyond its own is some other walk's, which carries it on to the ancestors), and
+// of equal bounds either zero's sign may stay. One lane walking for all of them took
+// 4.8 ms for 160 worlds of 50 to 4,000 bodies and 2.4 ms for 16,384 of 10 to 500.
+constexpr int kEnlargeLanes = 256;
+
+// aabbEnlarge's test and store of one bound, against other lanes; lower: a lower bound
+__device__ __forceinline__ bool growBound(float* bound, float v, bool lower) {
+  float cur = *reinterpret_cast<volatile float*>(bound);
+  while (lower ? v < cur : cur < v) {
+    const int seen = __float_as_int(cur);
+    const int old = atomicCAS(reinterpret_cast<int*>(bound), seen, __float_as_int(v));
+    if (old == seen) return true;
+    cur = __int_as_float(old);
+  }
+  return false;
+}
+
+__global__ __launch_bounds__(kEnlargeLanes) void enlargePendingKernel(BatchView b) {
   const int world = blockIdx.x;
-  WorldHeader* h = b.worlds + world;
+  const WorldHeader* h = b.worlds + world;
   Shape* shapes = b.shapes + h->shapeOffset;
   const int ns = h->shapeCount;
-  bool any = false;
-  for (int k = threadIdx.x; k < ns; k += 64) any |= (shapes[k].flags & SF_TREE_PENDING) != 0;
-  if (!__syncthreads_or(any) || threadIdx.x != 0) return;
-  for (int k = 0; k < ns; ++k) {
+  for (int k = threadIdx.x; k < ns; k += kEnlargeLanes) {
     Shape& sh = shapes[k];
-    if (!(sh.flags & SF_TREE_PENDING)) continue;
+    const int flags = sh.flags;
+    if (!(flags & SF_TREE_PENDING)) continue;
     const int t = sh.proxyKey & 3;
     if (sh.proxyKey < 0 || t == kStatic) continue;
-    TreeHeader* hd = b.treeHdrs + 3L * world + t;
+    const TreeHeader* hd = b.treeHdrs + 3L * world + t;
     TreeNode* n = b.treeNodes + hd->offset;
     const int F = hd->fresh;
     const int leaf = sh.proxyKey >> 2;
     if (leaf < 0 || leaf >= F) continue;  // left to the tree launch, which flags the tree
-    sh.flags &= ~SF_TREE_PENDING;
+    sh.flags = flags & ~SF_TREE_PENDING;
     const AABB box = sh.fat;
     n[leaf].box = box;
-    int p = n[leaf].parent;
-    for (int g = 0; p >= 0 && p < F && g < F; ++g) {
-      const bool changed = aabbEnlarge(&n[p].box, box);
-      n[p].flags |= TN_ENLARGED;
-      p = n[p].parent;
-      if (!changed) break;
-    }
-    for (int g = 0; p >= 0 && p < F && g < F; ++g) {
-      if (n[p].flags & TN_ENLARGED) break;
-      n[p].flags |= TN_ENLARGED;
-      p = n[p].parent;
+    bool grow = true, mark = true;
+    for (int p = n[leaf].parent, g = 0; p >= 0 && p < F && g < F && (grow || mark); p = n[p].parent, ++g) {
+      // the flags share a word with the height, which no launch changes beside this one
+      if (mark) {
+        const uint32_t old = atomicOr(reinterpret_cast<uint32_t*>(&n[p].height), (uint32_t)TN_ENLARGED << 16);
+        mark = ((old >> 16) & TN_ENLARGED) == 0;
+      }
+      if (grow) {
+        AABB* a = &n[p].box;
+        const bool lx = growBound(&a->lo.x, box.lo.x, true), ly = growBound(&a->lo.y, box.lo.y, true);
+        const bool hx = growBound(&a->hi.x, box.hi.x, false), hy = growBound(&a->hi.y, box.hi.y, false);
+        grow = lx || ly || hx || hy;
+      }
     }
   }
 }
@@ -2860,7 +2877,8 @@ __global__ void zeroIntsKernel(int* p, int n) {
 // walk them).
 extern "C" int f2d_launch_enlarge_pending(const f2d::BatchView* b, hipStream_t stream) {
   if (b->worldCount <= 0) return 0;
-  hipLaunchKernelGGL(f2d::enlargePendingKernel, dim3((unsigned)b->worldCount), dim3(64), 0, stream, *b);
+  hipLaunchKernelGGL(f2d::enlargePendingKernel, dim3((unsigned)b->worldCount), dim3(f2d::kEnlargeLanes), 0,
+                     stream, *b);
   return (int)hipGetLastError();
 }
 
