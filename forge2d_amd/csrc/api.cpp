@@ -1896,6 +1896,8 @@ static int importWorld(HostWorld& hw, const unsigned char* buf, long bytes, std:
     c.shapeA = sc.shape_a;
     c.shapeB = sc.shape_b;
     c.flags = sc.flags & (CF_TOUCHING | CF_CONTACT_EVENTS);
+    if (c.shapeA < (int)hw.geoms.size() && c.shapeB >= 0 && c.shapeB < (int)hw.geoms.size())
+      c.flags |= manifoldKind(hw.geoms[c.shapeA].type, hw.geoms[c.shapeB].type) << CF_KIND_SHIFT;
     c.simFlags = sc.sim_flags & (SIM_TOUCHING | SIM_HIT_EVENT | SIM_PRESOLVE);
     c.color = sc.color;
     c.friction = sc.friction;
@@ -2136,10 +2138,10 @@ long f2dg_device_bytes(void* h) {
 
 // Step every world of the batch `steps` times: one launch per step, one workgroup per world.
 // Lane candidates of a size class for online tuning: 64, 128 and 256 lanes per
-// world, 128, 256 and 512 for worlds of more than 128 shapes or bodies, 256, 512 and
-// 1024 for worlds of more than 512.
+// world, 256, 512 and 1024 for worlds of more than 512 shapes or bodies.
 static int laneCandidate(const SizeClass& c, int k) {
-  return (c.limit > 512 ? 256 : c.limit > 128 ? 128 : 64) << k;
+  static const int small[3] = {64, 128, 256}, large[3] = {256, 512, 1024};
+  return c.limit > 512 ? large[k] : small[k];
 }
 
 // One online tuning round: three steps, step k with every class at its k-th lane

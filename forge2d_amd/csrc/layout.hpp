@@ -47,6 +47,8 @@ enum : int {
   CF_CONTACT_EVENTS = 0x4,  // b2_contactEnableContactEvents (0x2 is the unused hit-event flag)
   CF_OFF_AWAKE = 0x100,     // not in the awake set (disabled or sleeping set): not collided
   CF_REF_MASK = 0x7,        // the bits that are the reference's b2ContactFlags
+  CF_KIND_SHIFT = 12,       // the pair's ManifoldKind, three bits
+  CF_KIND_MASK = 0x7,
   SIM_TOUCHING = 0x00010000,
   SIM_DISJOINT = 0x00020000,
   SIM_STARTED = 0x00040000,

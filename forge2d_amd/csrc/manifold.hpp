@@ -681,41 +681,43 @@ F2D_HD bool isPrimary(int ta, int tb) {
   return ta > tb;
 }
 
+// The manifold code a pair of shape types (in registered order) runs. Segments share the
+// capsule code with radius 0 and the polygon code with a two-vertex polygon, as do capsules
+// against polygons, so the nine registered pairs run five bodies of code.
+enum ManifoldKind : int {
+  kCirclesManifold = 0,
+  kCapsuleCircleManifold,
+  kCapsulesManifold,
+  kPolygonCircleManifold,
+  kPolygonsManifold,
+  kManifoldKinds
+};
+F2D_HD int manifoldKind(int ta, int tb) {
+  if (tb == kCircle) return ta == kCircle ? kCirclesManifold
+                                          : (ta == kPolygon ? kPolygonCircleManifold : kCapsuleCircleManifold);
+  return ta != kPolygon && tb == kCapsule ? kCapsulesManifold : kPolygonsManifold;
+}
+
 // Dispatch, S/contact.c:67-149. Shapes are already in registered (primary) order.
-F2D_HD void computeManifold(Manifold& m, const ShapeGeom& gA, Xf xfA, const ShapeGeom& gB, Xf xfB) {
-  int ta = gA.type, tb = gB.type;
-  if (ta == kCircle) {  // circle-circle
+F2D_HD void computeManifold(Manifold& m, int kind, const ShapeGeom& gA, Xf xfA, const ShapeGeom& gB, Xf xfB) {
+  const float radiusA = gA.type == kSegment ? 0.0f : gA.radius;
+  if (kind == kCirclesManifold) {
     collideCircles(m, gA.v[0], gA.radius, xfA, gB.v[0], gB.radius, xfB);
-  } else if (ta == kCapsule) {
-    if (tb == kCircle) {
-      collideCapsuleAndCircle(m, gA.v[0], gA.v[1], gA.radius, xfA, gB.v[0], gB.radius, xfB);
-    } else {
-      collideCapsules(m, gA.v[0], gA.v[1], gA.radius, xfA, gB.v[0], gB.v[1], gB.radius, xfB);
-    }
-  } else if (ta == kPolygon) {
+  } else if (kind == kCapsuleCircleManifold) {
+    collideCapsuleAndCircle(m, gA.v[0], gA.v[1], radiusA, xfA, gB.v[0], gB.radius, xfB);
+  } else if (kind == kCapsulesManifold) {
+    collideCapsules(m, gA.v[0], gA.v[1], radiusA, xfA, gB.v[0], gB.v[1], gB.radius, xfB);
+  } else if (kind == kPolygonCircleManifold) {
     Poly A;
     loadPoly(A, gA);
-    if (tb == kCircle) {
-      collidePolygonAndCircle(m, A, xfA, gB.v[0], gB.radius, xfB);
-    } else if (tb == kCapsule) {
-      Poly B = makeCapsulePoly(gB.v[0], gB.v[1], gB.radius);
-      collidePolygons(m, A, xfA, B, xfB);
-    } else {
-      Poly B;
-      loadPoly(B, gB);
-      collidePolygons(m, A, xfA, B, xfB);
-    }
-  } else {  // segment A
-    if (tb == kCircle) {
-      collideCapsuleAndCircle(m, gA.v[0], gA.v[1], 0.0f, xfA, gB.v[0], gB.radius, xfB);
-    } else if (tb == kCapsule) {
-      collideCapsules(m, gA.v[0], gA.v[1], 0.0f, xfA, gB.v[0], gB.v[1], gB.radius, xfB);
-    } else {
-      Poly A = makeCapsulePoly(gA.v[0], gA.v[1], 0.0f);
-      Poly B;
-      loadPoly(B, gB);
-      collidePolygons(m, A, xfA, B, xfB);
-    }
+    collidePolygonAndCircle(m, A, xfA, gB.v[0], gB.radius, xfB);
+  } else {
+    Poly A, B;
+    if (gA.type == kPolygon) loadPoly(A, gA);
+    else A = makeCapsulePoly(gA.v[0], gA.v[1], radiusA);
+    if (gB.type == kPolygon) loadPoly(B, gB);
+    else B = makeCapsulePoly(gB.v[0], gB.v[1], gB.radius);
+    collidePolygons(m, A, xfA, B, xfB);
   }
 }
 

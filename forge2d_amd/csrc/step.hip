@@ -384,6 +384,7 @@ __device__ void createContacts(const WorldPtrs& w, SharedState& sh, uint64_t* pk
           atomicOr(&h->error, ERR_CONTACT_CAP);
         }
       }
+      const int kind = valid ? manifoldKind(w.geoms[a].type, w.geoms[bsh].type) : 0;
       pk[i] = ((uint64_t)(uint32_t)a << 32) | (uint32_t)bsh;
       pv[i] = id;
       if (id >= 0) {
@@ -392,7 +393,7 @@ __device__ void createContacts(const WorldPtrs& w, SharedState& sh, uint64_t* pk
         Contact& c = w.contacts[id];
         c.shapeA = a;
         c.shapeB = bsh;
-        c.flags = ((A.flags | B.flags) & SF_CONTACT_EVENTS) ? CF_CONTACT_EVENTS : 0;
+        c.flags = (((A.flags | B.flags) & SF_CONTACT_EVENTS) ? CF_CONTACT_EVENTS : 0) | (kind << CF_KIND_SHIFT);
         c.simFlags = ((A.flags | B.flags) & SF_PRESOLVE) ? SIM_PRESOLVE : 0;
         c.color = -1;
         c.localIndex = -1;
@@ -476,7 +477,9 @@ __device__ __forceinline__ int sweepShape(const WorldPtrs& w, const float4* boxe
 // Every sweep of a workgroup's shapes [first, first + count): each lane sweeps its
 // shapes up to kLongRun candidates; longer sweeps are continued by all lanes, one
 // after another, each lane testing every BLOCK-th candidate (the sorted boxes end
-// a lane's part at the first box past the shape's upper x). Every (i, j) candidate
+// a lane's part at the first box past the shape's upper x), or, from two for every
+// wavefront on, by a wavefront each: a stack's columns hand over hundreds of sweeps of
+// some fifty candidates more (an 820-box pyramid: 256, 395 k cycles one after another). Every (i, j) candidate
 // is tested exactly once; the pairs' order is fixed later by their sort.
 template <int BLOCK>
 __device__ void sweepShapes(const WorldPtrs& w, LongSweeps& sh, const float4* boxes, const int* order,
@@ -499,9 +502,17 @@ __device__ void sweepShapes(const WorldPtrs& w, LongSweeps& sh, const float4* bo
   }
   __syncthreads();
   const int nLong = min(sh.count, kLongSweeps);
-  for (int k = 0; k < nLong; ++k) {
-    const int i = sh.shape[k];
-    sweepShape(w, boxes, order, info, i, sh.next[k] + threadIdx.x, BLOCK, n, -1, pairCount, pairSet, pairMask);
+  constexpr int kWaves = BLOCK / 64;
+  if (nLong < 2 * kWaves) {
+    for (int k = 0; k < nLong; ++k) {
+      const int i = sh.shape[k];
+      sweepShape(w, boxes, order, info, i, sh.next[k] + threadIdx.x, BLOCK, n, -1, pairCount, pairSet, pairMask);
+    }
+  } else {
+    for (int k = threadIdx.x >> 6; k < nLong; k += kWaves) {
+      const int i = sh.shape[k];
+      sweepShape(w, boxes, order, info, i, sh.next[k] + (threadIdx.x & 63), 64, n, -1, pairCount, pairSet, pairMask);
+    }
   }
   __syncthreads();
 }
@@ -675,7 +686,7 @@ __device__ void updateContact(const WorldPtrs& w, Contact& c) {
   bool wasTouching = (c.simFlags & SIM_TOUCHING) != 0;
   Manifold old = c.m;
   Manifold m;
-  computeManifold(m, w.geoms[c.shapeA], xfA, w.geoms[c.shapeB], xfB);
+  computeManifold(m, (c.flags >> CF_KIND_SHIFT) & CF_KIND_MASK, w.geoms[c.shapeA], xfA, w.geoms[c.shapeB], xfB);
   c.friction = sqrtf(A.friction * B.friction);
   c.restitution = maxf(A.restitution, B.restitution);
   if (A.rollingResistance > 0.0f || B.rollingResistance > 0.0f) {
@@ -741,28 +752,97 @@ __device__ void updateContact(const WorldPtrs& w, Contact& c) {
   c.m = m;
 }
 
-// The narrow phase of contact slot i: awake contacts whose fat boxes stopped
-// overlapping are flagged disjoint, the others get a new manifold.
-__device__ __forceinline__ void collideContact(const WorldPtrs& w, int i) {
+// What the narrow phase does with contact slot i: nothing (-1), flag it disjoint (done here,
+// -1) when its fat boxes stopped overlapping, or a new manifold of the returned kind.
+// Only the awake set collides (S/world.c:496-521).
+__device__ __forceinline__ int narrowKind(const WorldPtrs& w, int i) {
   Contact& c = w.contacts[i];
-  if (c.shapeA < 0 || (c.flags & CF_OFF_AWAKE)) return;  // only the awake set collides (S/world.c:496-521)
-  AABB fa = w.shapes[c.shapeA].fat, fb = w.shapes[c.shapeB].fat;
-  if (!aabbOverlaps(fa, fb)) {
-    c.simFlags |= SIM_DISJOINT;
-    c.simFlags &= ~SIM_TOUCHING;
-  } else {
-    updateContact(w, c);
+  const int sa = c.shapeA, flags = c.flags;
+  if (sa < 0 || (flags & CF_OFF_AWAKE)) return -1;
+  const AABB fa = w.shapes[sa].fat, fb = w.shapes[c.shapeB].fat;
+  if (aabbOverlaps(fa, fb)) return (flags >> CF_KIND_SHIFT) & CF_KIND_MASK;
+  c.simFlags = (c.simFlags | SIM_DISJOINT) & ~SIM_TOUCHING;
+  return -1;
+}
+
+struct NarrowBins {
+  int count[kManifoldKinds], start[kManifoldKinds], fill[kManifoldKinds];
+  int runs;  // wavefront runs of one kind
+};
+
+// The narrow phase of contact slots [first, first + n) on one workgroup. The slots are
+// gathered by manifold kind, and every wavefront then takes runs of 64 contacts of one
+// kind: the five kinds' code differs by up to ten times in length, and a wavefront of
+// mixed kinds ran all of it. Contacts update independently, so their order is free.
+// ldsBytes at `lds`: five bytes a slot, else the slots are taken as they come.
+template <int BLOCK>
+__device__ __forceinline__ void narrowPhase(const WorldPtrs& w, NarrowBins& bins, char* lds, int ldsBytes, int first,
+                                            int n) {
+  if (5L * n > (long)ldsBytes) {
+    for (int k = threadIdx.x; k < n; k += BLOCK)
+      if (narrowKind(w, first + k) >= 0) updateContact(w, w.contacts[first + k]);
+    return;
+  }
+  int* list = reinterpret_cast<int*>(lds);
+  signed char* kinds = reinterpret_cast<signed char*>(lds + 4L * n);
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x < kManifoldKinds) bins.count[threadIdx.x] = bins.fill[threadIdx.x] = 0;
+  __syncthreads();
+  for (int base = 0; base < n; base += BLOCK) {
+    const int k = base + threadIdx.x;
+    const int kind = k < n ? narrowKind(w, first + k) : -1;
+    if (k < n) kinds[k] = (signed char)kind;
+    F2D_UNROLL
+    for (int t = 0; t < kManifoldKinds; ++t) {
+      const int c = __popcll(__ballot(kind == t));
+      if (lane == 0 && c > 0) atomicAdd(&bins.count[t], c);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int s = 0, runs = 0;
+    F2D_UNROLL
+    for (int t = 0; t < kManifoldKinds; ++t) {
+      bins.start[t] = s;
+      s += bins.count[t];
+      runs += (bins.count[t] + 63) >> 6;
+    }
+    bins.runs = runs;
+  }
+  __syncthreads();
+  for (int base = 0; base < n; base += BLOCK) {
+    const int k = base + threadIdx.x;
+    const int kind = k < n ? kinds[k] : -1;
+    F2D_UNROLL
+    for (int t = 0; t < kManifoldKinds; ++t) {
+      const unsigned long long m = __ballot(kind == t);
+      int at = 0;
+      if (lane == 0 && m != 0ull) at = atomicAdd(&bins.fill[t], __popcll(m));
+      at = __shfl(at, 0, 64);
+      if (kind == t) list[bins.start[t] + at + __popcll(m & laneMaskLt(lane))] = first + k;
+    }
+  }
+  __syncthreads();
+  // the longest code (polygons, the last kind) first
+  for (int r = threadIdx.x >> 6; r < bins.runs; r += BLOCK / 64) {
+    int t = kManifoldKinds - 1, run = r;
+    for (; t > 0; --t) {
+      const int mine = (bins.count[t] + 63) >> 6;
+      if (run < mine) break;
+      run -= mine;
+    }
+    const int k = run * 64 + lane;
+    if (k < bins.count[t]) updateContact(w, w.contacts[list[bins.start[t] + k]]);
   }
 }
 
 // contactsDone: a narrow-phase launch already updated the contacts
 template <int BLOCK>
-__device__ void collidePhase(const WorldPtrs& w, SharedState& sh, bool contactsDone) {
+__device__ void collidePhase(const WorldPtrs& w, SharedState& sh, NarrowBins& bins, char* lds, int ldsBytes,
+                             bool contactsDone) {
   WorldHeader* h = w.hdr;
   const int n = h->contactCount;
-  if (!contactsDone) {
-    for (int i = threadIdx.x; i < n; i += BLOCK) collideContact(w, i);
-  }
+  if (!contactsDone) narrowPhase<BLOCK>(w, bins, lds, ldsBytes, 0, n);
   __syncthreads();
   // ordered list of contacts whose state changed (ascending contact id)
   if (threadIdx.x == 0) sh.changedCount = 0;
@@ -1896,6 +1976,7 @@ template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void collideKernel(BatchView b, StepParams sp, const int* worldList, int ldsBytes) {
   __shared__ SharedState sh;
   __shared__ WorldPtrs serialW;
+  __shared__ NarrowBins bins;
   extern __shared__ __align__(16) char lds[];
   const int wi = worldList ? worldList[blockIdx.x] : blockIdx.x;
   WorldHeader* h = b.worlds + wi;
@@ -1920,7 +2001,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   } else if (sp.phases & PH_PAIRS_FINISH) {
     pairsPhase<BLOCK>(w, sh, lds, ldsShapes, ldsPairs, ldsBytes, 2);
   }
-  if (sp.phases & PH_COLLIDE) collidePhase<BLOCK>(w, sh, (sp.phases & PH_CONTACTS_DONE) != 0);
+  if (sp.phases & PH_COLLIDE) collidePhase<BLOCK>(w, sh, bins, lds, ldsBytes, (sp.phases & PH_CONTACTS_DONE) != 0);
   if (sp.phases & PH_STATE) statePhase<BLOCK>(w, sh, serialW, lds, ldsBytes);
   if (threadIdx.x == 0 && (sp.phases & (PH_SOLVE | PH_FINALIZE | PH_NO_COUNT)) == 0) h->stepIndex += 1;
 }
@@ -1941,21 +2022,26 @@ __global__ __launch_bounds__(256) void sweepKernel(BatchView b, const int* world
                    nullptr, 0u);
 }
 
-// Solver stages and finalize of one world per workgroup; body states and the
-// per-step body terms live in ldsBytes of dynamic LDS (64 B per body) when they fit.
 // The narrow phase of the worlds of a split pair update: workgroup blockIdx.x of
-// gridDim.x takes every gridDim.x-th run of 256 contact slots of world blockIdx.y
+// gridDim.x takes every gridDim.x-th run of kNarrowChunk contact slots of world blockIdx.y
 // (contacts update independently; the collide launch after it lists the changes).
+constexpr int kNarrowChunk = 512;  // enough for full wavefronts of the common kinds
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void narrowKernel(BatchView b,
                                                                                             const int* worldList) {
+  __shared__ NarrowBins bins;
+  __shared__ __align__(16) char lds[5 * kNarrowChunk];
   const int wi = worldList ? worldList[blockIdx.y] : blockIdx.y;
   WorldHeader* h = b.worlds + wi;
   const int n = h->contactCount;
-  if ((int)blockIdx.x * 256 >= n) return;
+  if ((int)blockIdx.x * kNarrowChunk >= n) return;
   WorldPtrs w = worldPtrs(b, h);
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) collideContact(w, i);
+  for (int first = blockIdx.x * kNarrowChunk; first < n; first += gridDim.x * kNarrowChunk) {
+    narrowPhase<256>(w, bins, lds, 5 * kNarrowChunk, first, min(kNarrowChunk, n - first));
+    __syncthreads();
+  }
 }
 
+// Solver stages and finalize of one world per workgroup.
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void solveKernel(BatchView b, StepParams sp, const int* worldList, int ldsBytes) {
   __shared__ SharedState sh;
