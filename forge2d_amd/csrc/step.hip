@@ -503,16 +503,11 @@ __device__ void sweepShapes(const WorldPtrs& w, LongSweeps& sh, const float4* bo
   __syncthreads();
   const int nLong = min(sh.count, kLongSweeps);
   constexpr int kWaves = BLOCK / 64;
-  if (nLong < 2 * kWaves) {
-    for (int k = 0; k < nLong; ++k) {
-      const int i = sh.shape[k];
-      sweepShape(w, boxes, order, info, i, sh.next[k] + threadIdx.x, BLOCK, n, -1, pairCount, pairSet, pairMask);
-    }
-  } else {
-    for (int k = threadIdx.x >> 6; k < nLong; k += kWaves) {
-      const int i = sh.shape[k];
-      sweepShape(w, boxes, order, info, i, sh.next[k] + (threadIdx.x & 63), 64, n, -1, pairCount, pairSet, pairMask);
-    }
+  const bool together = nLong < 2 * kWaves;
+  const int lane = together ? threadIdx.x : threadIdx.x & 63, step = together ? BLOCK : 64;
+  for (int k = together ? 0 : threadIdx.x >> 6; k < nLong; k += together ? 1 : kWaves) {
+    const int i = sh.shape[k];
+    sweepShape(w, boxes, order, info, i, sh.next[k] + lane, step, n, -1, pairCount, pairSet, pairMask);
   }
   __syncthreads();
 }
@@ -1973,7 +1968,7 @@ __device__ void stepContext(const WorldHeader* h, const StepParams& sp, SolveCtx
 // Four waves per SIMD: the compiler keeps the manifold code within 128 VGPRs
 // (measured faster than the 148-VGPR, three-wave build on the 16k-world workload).
 template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void collideKernel(BatchView b, StepParams sp, const int* worldList, int ldsBytes) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void collideKernel(BatchView b, StepParams sp, const int* worldList, int ldsBytes) {
   __shared__ SharedState sh;
   __shared__ WorldPtrs serialW;
   __shared__ NarrowBins bins;
@@ -2026,7 +2021,7 @@ __global__ __launch_bounds__(256) void sweepKernel(BatchView b, const int* world
 // gridDim.x takes every gridDim.x-th run of kNarrowChunk contact slots of world blockIdx.y
 // (contacts update independently; the collide launch after it lists the changes).
 constexpr int kNarrowChunk = 512;  // enough for full wavefronts of the common kinds
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void narrowKernel(BatchView b,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void narrowKernel(BatchView b,
                                                                                             const int* worldList) {
   __shared__ NarrowBins bins;
   __shared__ __align__(16) char lds[5 * kNarrowChunk];
