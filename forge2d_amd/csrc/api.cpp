@@ -31,6 +31,8 @@ extern "C" int f2d_launch_step(const f2d::BatchView* b, const f2d::StepParams* s
 extern "C" int f2d_launch_island_command(const f2d::BatchView* b, int world, int op, int arg, hipStream_t stream);
 extern "C" int f2d_launch_queries(const f2d::BatchView* b, int* group, const f2d::Query* q, int n,
                                   f2d::QueryHit* hits, int* counts, int cap, hipStream_t stream);
+extern "C" int f2d_launch_frame(const f2d::BatchView* b, int world, int bodyCap, int* head,
+                                f2d::FrameRecord* records, hipStream_t stream);
 extern "C" int f2d_launch_enlarge_pending(const f2d::BatchView* b, hipStream_t stream);
 extern "C" int f2d_launch_explosions(const f2d::BatchView* b, const f2d::Query* q, int n, hipStream_t stream);
 
@@ -1238,6 +1240,12 @@ static int upload(Batch& b) {
   return 0;
 }
 
+// The device state moved on: the mirror is stale and the last frame's records are over.
+static void deviceStepped(Batch& b) {
+  b.deviceNewer = true;
+  b.frameFresh = false;
+}
+
 // Copy the device state of every world back to the host mirror: one copy per flat
 // array, then a scatter into the worlds' vectors.
 static int download(Batch& b) {
@@ -1324,6 +1332,7 @@ static int download(Batch& b) {
     hw.inv_h = h.inv_h;
   }
   b.deviceNewer = false;
+  b.frameFresh = false;
   return 0;
 }
 
@@ -2084,6 +2093,7 @@ void f2dg_destroy(void* h) {
   Batch* b = static_cast<Batch*>(h);
   if (!b) return;
   freeDevice(*b);
+  if (b->frame) (void)hipHostFree(b->frame);
   if (b->ownsStream && b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
 }
@@ -2203,7 +2213,7 @@ int f2dg_step(void* h, float dt, int subSteps, int steps, int phases) {
     ++s;
     if (b->tunePeriod > 0) ++b->tuneClock;
   }
-  b->deviceNewer = true;
+  deviceStepped(*b);
   return 0;
 }
 
@@ -2235,7 +2245,7 @@ int f2dg_step_worlds(void* h, const int* worldIds, int n, float dt, int subSteps
     for (int s = 0; s < steps; ++s) {
       if (f2d_launch_step(&b->dev.view, &sp, b->dWorldList, n, b->stream, &b->launch) != 0) return -1;
     }
-    b->deviceNewer = true;
+    deviceStepped(*b);
     return 0;
   }
   // the listed worlds grouped by size class, each group with its class's launch
@@ -2262,7 +2272,7 @@ int f2dg_step_worlds(void* h, const int* worldIds, int n, float dt, int subSteps
     for (int k = 0; k < K; ++k)
       if (start[k + 1] > start[k]) F2D_HIP(hipStreamWaitEvent(b->stream, b->classes[k].done, 0));
   }
-  b->deviceNewer = true;
+  deviceStepped(*b);
   return 0;
 }
 
@@ -2282,7 +2292,7 @@ int f2dg_step_each(void* h, float dt, int subSteps, int steps) {
       if (f2d_launch_step(&b->dev.view, &sp, b->dWorldList + i, 1, b->stream, &b->launch) != 0) return -1;
     }
   }
-  b->deviceNewer = true;
+  deviceStepped(*b);
   return 0;
 }
 
@@ -2308,7 +2318,7 @@ int f2dg_step_timed(void* h, float dt, int subSteps, int steps, float* msOut) {
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   *msOut = ms;
-  b->deviceNewer = true;
+  deviceStepped(*b);
   return 0;
 }
 
@@ -2345,7 +2355,7 @@ int f2dg_kernel_times(void* h, float dt, int subSteps, int steps, float* ms) {
   }
   for (auto& e : ev) (void)hipEventDestroy(e);
   for (int k = 0; k < 4; ++k) ms[k] = sum[k];
-  b->deviceNewer = true;
+  deviceStepped(*b);
   return 0;
 }
 
@@ -2379,7 +2389,7 @@ int f2dg_phase_times(void* h, float dt, int subSteps, int steps, float* ms) {
   }
   for (auto& e : ev) (void)hipEventDestroy(e);
   for (int k = 0; k < 4; ++k) ms[k] = sum[k];
-  b->deviceNewer = true;
+  deviceStepped(*b);
   return 0;
 }
 
@@ -2575,6 +2585,21 @@ static int hitEvents(Batch& b, int world, double* out, uint32_t shapeWg) {
 // of that finalize (S/solver.c:605-610); fellAsleep marks the bodies whose island
 // went to sleep at the end of the step (S/solver_set.c:196-205).
 static int bodyEvents(Batch& b, int world, double* out, int worldIndex0) {
+  if (b.frameFresh && b.deviceNewer) {  // a single world, straight after its step
+    const HostWorld& hw = b.worlds[world];
+    const int n = b.frame[1];
+    const FrameRecord* f = b.frameRecords();
+    for (int k = 0; out && k < n; ++k, ++f, out += 7) {
+      out[0] = (double)f->body + 1;
+      out[1] = worldIndex0 < 0 ? 0.0 : (double)((uint32_t)worldIndex0 | ((uint32_t)hw.bodyGen[f->body] << 16));
+      out[2] = f->px;
+      out[3] = f->py;
+      out[4] = f->qc;
+      out[5] = f->qs;
+      out[6] = f->fellAsleep;
+    }
+    return n;
+  }
   download(b);
   HostWorld& hw = b.worlds[world];
   const int n = std::min(hw.hdr.moveBodyCount, (int)hw.moveOrder.size());
@@ -2715,7 +2740,7 @@ int f2dg_autotune(void* h, float dt, int subSteps, int steps, float* msOut) {
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  b->deviceNewer = true;
+  deviceStepped(*b);
   return b->classes.empty() ? b->launch.block : b->classes.back().launch.block;
 }
 
@@ -2849,6 +2874,24 @@ void f2d_destroy_world(uint32_t w) {
 
 int f2d_world_is_valid(uint32_t w) { return batchOf(w) != nullptr; }
 
+// Pinned host memory for a frame of the batch's one world, kept until the world grows or
+// is destroyed.
+static bool reserveFrame(Batch& b) {
+  const int bodies = (int)b.worlds[0].sims.size();
+  if (b.frame && bodies <= b.frameCap) return true;
+  if (b.frame) (void)hipHostFree(b.frame);
+  b.frame = nullptr;
+  b.frameCap = 0;
+  const int cap = bodies + bodies / 2 + 16;
+  if (hipHostMalloc(&b.frame, 2 * sizeof(int) + sizeof(FrameRecord) * (size_t)cap, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    b.frame = nullptr;
+    return false;
+  }
+  b.frameCap = cap;
+  return true;
+}
+
 // f2d_shim.c:147-149 -> b2World_Step
 void f2d_world_step(uint32_t w, float time_step, int sub_steps) {
   Batch* b = batchOf(w);
@@ -2872,12 +2915,15 @@ void f2d_world_step(uint32_t w, float time_step, int sub_steps) {
                  b->lastError.c_str());
     std::abort();
   }
+  const bool frame = reserveFrame(*b) && f2d_launch_frame(&b->dev.view, 0, b->frameCap, b->frame, b->frameRecords(),
+                                                          b->stream) == 0;
   hipError_t e = hipStreamSynchronize(b->stream);
   if (e != hipSuccess) {
     std::fprintf(stderr, "forge2d_amd: world step failed on the device: %s\n", hipGetErrorString(e));
     std::abort();
   }
-  const int bits = f2dg_error_bits(b);
+  b->frameFresh = frame;
+  const int bits = frame ? b->frame[0] : f2dg_error_bits(b);
   if (bits != 0) {
     std::fprintf(stderr, "forge2d_amd: world step exceeded a device capacity (error bits 0x%x:%s%s%s%s%s)\n", bits,
                  (bits & ERR_CONTACT_CAP) ? " contacts" : "", (bits & ERR_PAIR_CAP) ? " new pairs" : "",
@@ -2911,7 +2957,7 @@ static void islandCommand(Batch& b, int world, int op, int arg) {
   }
   if (f2d_launch_island_command(&b.dev.view, world, op, arg, b.stream) != 0) return;
   (void)hipStreamSynchronize(b.stream);
-  b.deviceNewer = true;
+  deviceStepped(b);
 }
 
 // b2World_EnableSleeping, S/world.c:1710-1737: disabling sleep wakes every sleeping set
@@ -4773,7 +4819,7 @@ static int runQueries(Batch& b, const Query* q, int n, QueryHit* hits, int* coun
   long used = 0;
   for (int i = 0; i < n; ++i) used = std::max<long>(used, (long)i * cap + std::min(std::max(counts[i], 0), cap));
   if (used > 0) F2D_HIP(hipMemcpy(hits, b.dHits, sizeof(QueryHit) * used, hipMemcpyDeviceToHost));
-  b.deviceNewer = true;  // pending tree enlargements applied, explosions
+  deviceStepped(b);  // pending tree enlargements applied, explosions
   return 0;
 }
 
@@ -4811,7 +4857,7 @@ int f2dg_query_device(void* h, const void* queries, int n, void* hits, void* cou
     if (upload(*b) != 0) return -1;
   }
   if (ensureGroupBuffer(*b, n) != 0) return -1;
-  b->deviceNewer = true;  // pending tree enlargements applied
+  deviceStepped(*b);  // pending tree enlargements applied
   return f2d_launch_queries(&b->dev.view, b->dGroup, static_cast<const Query*>(queries), n,
                             static_cast<QueryHit*>(hits), static_cast<int*>(counts), cap, b->stream);
 }

@@ -345,6 +345,13 @@ struct QueryHit {
 };
 static_assert(sizeof(Query) == 48 && sizeof(QueryHit) == 24, "query records");
 
+// One moved body of a frame (f2d_world_step), in pinned host memory
+struct FrameRecord {
+  int body;
+  float px, py, qc, qs;
+  int fellAsleep;
+};
+
 // Launch shape of a batch: workgroup size and dynamic LDS bytes per kernel.
 // HBM work region of tree t of a world whose node region starts at `offset`
 F2D_HD long treeWorkOffset(int offset, int world, int t) { return 25L * offset + 160L * (3L * world + t); }

@@ -112,6 +112,12 @@ struct Batch {
   bool committed = false;
   bool hostDirty = true;     // host holds changes the device lacks
   bool deviceNewer = false;  // device holds a step the host mirror lacks
+  // the last f2d_world_step's error bits and moved bodies: two ints, then records. Fresh
+  // until anything else steps, reads back or edits the world.
+  int* frame = nullptr;
+  int frameCap = 0;
+  bool frameFresh = false;
+  FrameRecord* frameRecords() const { return reinterpret_cast<FrameRecord*>(frame + 2); }
   hipStream_t stream = nullptr;
   bool ownsStream = false;
   int* dWorldList = nullptr;

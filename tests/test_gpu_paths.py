@@ -4,6 +4,7 @@ A world is a container of bodies whose shapes are a fixture's, so that their geo
 records are the reference's own; every step is compared as tests/test_gpu_oracle.py
 compares it, bit for bit, with the oracle stepping the device's previous state.
 """
+import ctypes
 import os
 
 import numpy as np
@@ -14,6 +15,7 @@ from forge2d_amd import scenes
 from forge2d_amd import snapshot as S
 from oracle import pyoracle as O
 from tests.conftest import GOLDEN, load_fixture
+from tests.flat_util import FlatWorld
 from tests.test_gpu_oracle import compare
 
 pytestmark = pytest.mark.gpu
@@ -85,3 +87,30 @@ def test_solver_stages(gpu, bodies, block, steps):
     b = F.Batch(spec)
     b.set_block(block)
     follow(spec, geoms, steps, b)
+
+
+# a frame's body events come from records written behind the step, or, once the mirror was
+# read back, from the mirror: the same, for worlds around the record kernel's 256 lanes
+@pytest.mark.parametrize("bodies,sleep,steps", [(1, True, 90), (255, False, 4), (256, True, 4), (700, False, 4)])
+def test_frame_records(gpu, bodies, sleep, steps):
+    L = F.lib()
+    spec, _ = container(bodies, 41 + bodies, sleep=sleep, speed=1.0)
+    w = FlatWorld(spec)
+    a, b = np.zeros((bodies + 1, 7)), np.zeros((bodies + 1, 7))
+    pos = (ctypes.c_float * 2)()
+    asleep = 0
+    for k in range(steps):
+        w.step()
+        n = L.f2d_world_get_body_event_count(w.w)
+        assert L.f2d_world_get_body_events(w.w, a.ctypes.data_as(F._PD)) == n
+        L.f2d_body_get_position(*w.bodies[1], pos)  # reads the mirror back
+        assert L.f2d_world_get_body_events(w.w, b.ctypes.data_as(F._PD)) == n
+        assert np.array_equal(a[:n], b[:n])
+        asleep += int(a[:n, 6].sum())
+    assert asleep > 0 or not (sleep and bodies == 1)
+    # an edit between the step and the read shows, as it always did
+    w.step()
+    L.f2d_body_set_transform(*w.bodies[1], 3.0, 4.0, 1.0, 0.0)
+    n = L.f2d_world_get_body_events(w.w, a.ctypes.data_as(F._PD))
+    assert n == 0 or a[:n][a[:n, 0] == w.bodies[1][0]][0, 2:4].tolist() == [3.0, 4.0]
+    w.close()
