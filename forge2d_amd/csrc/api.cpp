@@ -881,9 +881,10 @@ static int treeLdsBytes(const HostWorld& hw, int limit) {
   return need <= limit ? (int)((need + 255) & ~255L) : 0;
 }
 
-// lanes of the tree launch: about two proxies per lane per pass
+// lanes of the tree launch: about two proxies per lane per pass. From 1,024 proxies on the
+// work arrays leave LDS soon (1,400), and the passes wait for L2 instead: more lanes.
 static int treeBlockFor(int proxies) {
-  return proxies <= 96 ? 64 : (proxies <= 192 ? 128 : (proxies <= 4096 ? 256 : 1024));
+  return proxies <= 96 ? 64 : (proxies <= 192 ? 128 : (proxies <= 1024 ? 256 : 1024));
 }
 
 static int commit(Batch& b) {
@@ -1011,7 +1012,7 @@ static int commit(Batch& b) {
   b.launch.treeLds = 0;
   int maxProxies = 0;
   for (const HostWorld& hw : b.worlds) {
-    b.launch.treeLds = std::max(b.launch.treeLds, treeLdsBytes(hw, kLdsLimit));
+    b.launch.treeLds = std::max(b.launch.treeLds, treeLdsBytes(hw, deviceLdsLimit()));
     maxProxies = std::max(maxProxies, std::max(hw.tree[kDynamic].proxyCount, hw.tree[kKinematic].proxyCount));
   }
   b.launch.treeBlock = treeBlockFor(maxProxies);
@@ -1073,7 +1074,7 @@ static int commit(Batch& b) {
       c.launch.treeLds = 0;
       int maxProxies = 0;
       for (int i : members[k]) {
-        c.launch.treeLds = std::max(c.launch.treeLds, treeLdsBytes(b.worlds[i], kLdsLimit));
+        c.launch.treeLds = std::max(c.launch.treeLds, treeLdsBytes(b.worlds[i], deviceLdsLimit()));
         maxProxies = std::max(maxProxies, std::max(b.worlds[i].tree[kDynamic].proxyCount,
                                                    b.worlds[i].tree[kKinematic].proxyCount));
       }

@@ -257,16 +257,14 @@ F2D_HD_COLD void mergeAwakeIslands(IslandCtx& c) {
 
 // The merges of mergeAwakeIslands once every awake island points at its root and
 // the children's bodies, contacts and joints carry their roots' ids (the solve
-// kernel does both on all lanes): children merge into their roots in reverse
-// awake order.
-F2D_HD_COLD void mergeAwakeChildren(IslandCtx& c) {
-  WorldHeader* h = c.h;
-  h->mergePending = 0;
-  for (int i = h->awakeIslandCount - 1; i >= 0; --i) {
-    int id = c.awakeIslands[i];
-    if (c.islands[id].parent == -1) continue;
-    mergeIsland(c, id, false);
-    destroyIsland(c, id);
+// kernel does both on all lanes) and the children are listed in c.seeds in reverse
+// awake order. A child has no children of its own then, and a removal moves the last
+// awake island into a place behind those still to come, so the list stays right.
+F2D_HD_COLD void mergeAwakeChildren(IslandCtx& c, int children) {
+  c.h->mergePending = 0;
+  for (int k = 0; k < children; ++k) {
+    mergeIsland(c, c.seeds[k], false);
+    destroyIsland(c, c.seeds[k]);
   }
 }
 

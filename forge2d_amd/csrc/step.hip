@@ -341,10 +341,12 @@ __device__ void considerPair(const WorldPtrs& w, int* pairCount, int s, int t, c
 // creation order), with the result of a serial loop over them: ids are the LIFO
 // pool's pops in creation order (free list top first, then fresh ids), so each pair's
 // id follows from its rank among the pairs that get a contact; the records are filled
-// in parallel and only the body contact-list prepends run serially, in pair order.
-// pk is reused for the oriented shapes and pv for the ids.
+// in parallel. pk is reused for the oriented shapes and pv for the ids. edges: LDS for
+// edgeCap edges of the body contact lists (it may lie over pk).
+constexpr int kLinkedPairs = 1024;
 template <int BLOCK>
-__device__ void createContacts(const WorldPtrs& w, SharedState& sh, uint64_t* pk, int* pv, int count) {
+__device__ void createContacts(const WorldPtrs& w, SharedState& sh, uint64_t* pk, int* pv, int count, int4* edges,
+                               int edgeCap) {
   WorldHeader* h = w.hdr;
   const int freeCount = h->freeCount, fresh = h->contactCount, cap = h->contactCap;
   int created = 0;
@@ -419,7 +421,49 @@ __device__ void createContacts(const WorldPtrs& w, SharedState& sh, uint64_t* pk
     const int used = min(created, freeCount + (cap - fresh));
     h->freeCount = freeCount - min(used, freeCount);
     h->contactCount = fresh + max(used - freeCount, 0);
-    // body contact lists: prepend each new contact to both bodies' lists in creation order
+  }
+  // body contact lists: prepend each new contact to both bodies' lists in creation order
+  if (count <= kLinkedPairs && 2 * count <= edgeCap) {
+    // Every edge finds the neighbours it gets in its body's list by looking through all
+    // new edges: the prepends one after another wait for each body's head in turn (0.2 ms
+    // for 250 pairs of a 20,000-body world); the search grows with the square of the count.
+    // An edge: body (-1: no contact), list key, the body's head before.
+    __syncthreads();
+    for (int k = threadIdx.x; k < 2 * count; k += BLOCK) {
+      const int id = pv[k >> 1];
+      const int body = id < 0 ? -1 : ((k & 1) ? w.contacts[id].bodyB : w.contacts[id].bodyA);
+      edges[k] = make_int4(body, (id << 1) | (k & 1), body < 0 ? -1 : w.sims[body].headContactKey, 0);
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < 2 * count; k += BLOCK) {
+      const int4 e = edges[k];
+      if (e.x < 0) continue;
+      int older = -1, newer = -1, edgesOfBody = 0;
+      for (int j = 0; j < 2 * count; ++j) {
+        if (edges[j].x != e.x) continue;
+        ++edgesOfBody;
+        if (j < k) older = j;
+        if (j > k && newer < 0) newer = j;
+      }
+      const int next = older >= 0 ? edges[older].y : e.z, prev = newer >= 0 ? edges[newer].y : -1;
+      Contact& c = w.contacts[e.y >> 1];
+      if (e.y & 1) {
+        c.prevB = prev;
+        c.nextB = next;
+      } else {
+        c.prevA = prev;
+        c.nextA = next;
+      }
+      if (older < 0 && e.z >= 0) {
+        Contact& hc = w.contacts[e.z >> 1];
+        if ((e.z & 1) == 0) hc.prevA = e.y; else hc.prevB = e.y;
+      }
+      if (newer < 0) {
+        w.sims[e.x].headContactKey = e.y;
+        w.sims[e.x].contactCount += edgesOfBody;
+      }
+    }
+  } else if (threadIdx.x == 0) {
     for (int i = 0; i < count; ++i) {
       const int id = pv[i];
       if (id < 0) continue;
@@ -660,7 +704,8 @@ __device__ void pairsPhase(const WorldPtrs& w, SharedState& sh, char* lds, int l
     }
     __syncthreads();
     bitonicSort<BLOCK>(pk, pv, pp);
-    createContacts<BLOCK>(w, sh, pk, pv, count);
+    createContacts<BLOCK>(w, sh, pk, pv, count, reinterpret_cast<int4*>(lds),
+                          (pairsInLds ? 8 * ldsPairs : ldsBytes) / (int)sizeof(int4));
   }
   __syncthreads();
   for (int i = threadIdx.x; i < n; i += BLOCK) w.shapes[i].flags &= ~SF_MOVED;
@@ -773,17 +818,13 @@ struct NarrowBins {
 template <int BLOCK>
 __device__ __forceinline__ void narrowPhase(const WorldPtrs& w, NarrowBins& bins, char* lds, int ldsBytes, int first,
                                             int n) {
-  if (5L * n > (long)ldsBytes) {
-    for (int k = threadIdx.x; k < n; k += BLOCK)
-      if (narrowKind(w, first + k) >= 0) updateContact(w, w.contacts[first + k]);
-    return;
-  }
+  const bool gathered = 5L * n <= (long)ldsBytes;
   int* list = reinterpret_cast<int*>(lds);
   signed char* kinds = reinterpret_cast<signed char*>(lds + 4L * n);
   const int lane = threadIdx.x & 63;
   if (threadIdx.x < kManifoldKinds) bins.count[threadIdx.x] = bins.fill[threadIdx.x] = 0;
   __syncthreads();
-  for (int base = 0; base < n; base += BLOCK) {
+  for (int base = 0; gathered && base < n; base += BLOCK) {
     const int k = base + threadIdx.x;
     const int kind = k < n ? narrowKind(w, first + k) : -1;
     if (k < n) kinds[k] = (signed char)kind;
@@ -802,10 +843,10 @@ __device__ __forceinline__ void narrowPhase(const WorldPtrs& w, NarrowBins& bins
       s += bins.count[t];
       runs += (bins.count[t] + 63) >> 6;
     }
-    bins.runs = runs;
+    bins.runs = gathered ? runs : (n + 63) >> 6;
   }
   __syncthreads();
-  for (int base = 0; base < n; base += BLOCK) {
+  for (int base = 0; gathered && base < n; base += BLOCK) {
     const int k = base + threadIdx.x;
     const int kind = k < n ? kinds[k] : -1;
     F2D_UNROLL
@@ -820,14 +861,21 @@ __device__ __forceinline__ void narrowPhase(const WorldPtrs& w, NarrowBins& bins
   __syncthreads();
   // the longest code (polygons, the last kind) first
   for (int r = threadIdx.x >> 6; r < bins.runs; r += BLOCK / 64) {
-    int t = kManifoldKinds - 1, run = r;
-    for (; t > 0; --t) {
-      const int mine = (bins.count[t] + 63) >> 6;
-      if (run < mine) break;
-      run -= mine;
+    int slot = -1;
+    if (gathered) {
+      int t = kManifoldKinds - 1, run = r;
+      for (; t > 0; --t) {
+        const int mine = (bins.count[t] + 63) >> 6;
+        if (run < mine) break;
+        run -= mine;
+      }
+      const int k = run * 64 + lane;
+      if (k < bins.count[t]) slot = list[bins.start[t] + k];
+    } else {
+      const int k = r * 64 + lane;
+      if (k < n && narrowKind(w, first + k) >= 0) slot = first + k;
     }
-    const int k = run * 64 + lane;
-    if (k < bins.count[t]) updateContact(w, w.contacts[list[bins.start[t] + k]]);
+    if (slot >= 0) updateContact(w, w.contacts[slot]);
   }
 }
 
@@ -1312,12 +1360,15 @@ struct SolveCtx {
 // b2MergeAwakeIslands (S/island.c:547-590): its first loop leaves every awake island
 // pointing at its root; here every lane walks its islands' parent chains read-only (a
 // chain read while other lanes shorten it still ends at the same root) and writes its
-// own island's root, then one lane merges in reverse awake order.
+// own island's root, all lanes list the children in reverse awake order, and one lane merges
+// those: looking for them among all awake islands was most of its time (20,000 islands, a
+// few children: 1.6 ms).
 template <int BLOCK>
 __device__ __forceinline__ bool solveIslands(const WorldPtrs& w, SharedState& sh) {
   WorldHeader* h = w.hdr;
   const int nb = h->bodyCount, nc = h->contactCount;
   const bool merge = h->mergePending != 0;
+  int children = 0;
   if (merge) {
     IslandCtx ic = w.isl;
     for (int i = threadIdx.x; i < h->awakeIslandCount; i += BLOCK) {
@@ -1349,11 +1400,22 @@ __device__ __forceinline__ bool solveIslands(const WorldPtrs& w, SharedState& sh
       const Island& is = ic.islands[id];
       if (is.parent != -1 && is.setIndex == kAwakeSet) w.joints[j].islandId = is.parent;
     }
+    // the seeds array is idle until a split
+    const int awake = h->awakeIslandCount;
+    for (int base = 0; base < awake; base += BLOCK) {
+      const int i = awake - 1 - base - (int)threadIdx.x;
+      const int id = i >= 0 ? ic.awakeIslands[i] : -1;
+      const bool child = id >= 0 && ic.islands[id].parent != -1;
+      int total;
+      const int slot = children + blockCompact<BLOCK>(child, sh.waveSums, &total);
+      if (child) ic.seeds[slot] = id;
+      children += total;
+    }
     __syncthreads();
   }
   if (threadIdx.x == 0) {
     IslandCtx ic = w.isl;
-    if (merge) mergeAwakeChildren(ic);
+    if (merge) mergeAwakeChildren(ic, children);
     sh.noAwake = h->awakeBodyCount == 0 ? 1 : 0;
     if (!sh.noAwake && h->splitIslandId != -1) splitIsland(ic, h->splitIslandId);
     if (!sh.noAwake) h->splitIslandId = -1;
