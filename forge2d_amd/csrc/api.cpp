@@ -1223,12 +1223,23 @@ static int upload(Batch& b) {
   for (SizeClass& c : b.classes) {
     c.launch.continuous = b.launch.continuous;
     c.launch.bulletLds = 0;
+    c.launch.islandLds = 0;
   }
   // LDS for the proxies that bullets sweep against (20 B per shape), only where some
   // world of a class has bullets: it costs the other classes workgroups per compute unit
   int bulletShapes = 0;
+  b.launch.islandLds = 0;
   for (size_t i = 0; i < b.worlds.size(); ++i) {
     const HostWorld& hw = b.worlds[i];
+    // an island split's arrays (16 B a body, its marks and joints) and its edges (32 B a body
+    // for two touching contacts each; a split with more edges keeps them in scratch)
+    if (hw.hdr.flags & WF_SLEEP) {
+      const long need = 52L * (long)hw.sims.size() + 24L * (long)hw.joints.size() + hw.hdr.contactCap / 8 + 512;
+      const int lds = (int)std::min<long>(need, deviceLdsLimit());
+      SizeClass& c = b.classes[b.classOf[i]];
+      c.launch.islandLds = std::max(c.launch.islandLds, lds);
+      b.launch.islandLds = std::max(b.launch.islandLds, lds);
+    }
     const bool bullets = std::any_of(hw.sims.begin(), hw.sims.end(), [](const BodySim& s) { return s.flags & BF_BULLET; });
     const int bytes = 20 * (int)hw.shapes.size();
     if (!bullets || bytes > 40960) continue;

@@ -368,6 +368,8 @@ struct LaunchConfig {
   int treeBlock;   // lanes of the tree launch (64, 128, 256 or 1024)
   int continuousChunks = 0;  // > 0: the non-bullet sweeps of each world spread over this many
                              // workgroups, then bullets and the sleep phase in a second launch
+  int islandLds = 0;         // > 0: some world sleeps, its islands split in a launch of their own
+                             // with this much LDS
   int bulletLds = 0;         // proxies in query order for bullets (0: no bullets, or worlds too large)
   int wideChunks = 0;        // > 0: the solve stages of each world as launches of this many
                              // 256-lane workgroups

@@ -114,3 +114,10 @@ def test_frame_records(gpu, bodies, sleep, steps):
     n = L.f2d_world_get_body_events(w.w, a.ctypes.data_as(F._PD))
     assert n == 0 or a[:n][a[:n, 0] == w.bodies[1][0]][0, 2:4].tolist() == [3.0, 4.0]
     w.close()
+
+
+# islands split on all lanes, their edges in LDS or (above 1,024 bodies) in the scratch region
+@pytest.mark.parametrize("bodies,steps", [(40, 200), (300, 150), (1500, 100)])
+def test_islands_sleep_and_split(gpu, bodies, steps):
+    spec, geoms = container(bodies, 7 + bodies, sleep=True, speed=1.0)
+    follow(spec, geoms, steps)
