@@ -366,6 +366,10 @@ struct LaunchConfig {
                    // narrow-phase launch over many workgroups
   int treeLds;     // tree rebuild work arrays (worlds whose trees need more use HBM)
   int treeBlock;   // lanes of the tree launch (64, 128, 256 or 1024)
+  hipStream_t treeStream = nullptr;  // the tree launch runs here, beside the contacts and the
+                                     // solve (null: in order)
+  hipEvent_t treeFork = nullptr, treeDone = nullptr;
+  int treeMarkChunks = 0;    // workgroups per world of the launch before it
   int continuousChunks = 0;  // > 0: the non-bullet sweeps of each world spread over this many
                              // workgroups, then bullets and the sleep phase in a second launch
   int islandLds = 0;         // > 0: some world sleeps, its islands split in a launch of their own

@@ -222,11 +222,11 @@ __device__ __forceinline__ int blockInclusiveMax(int v, int* sums, int* total) {
 
 // One tree of one world: the leaves the last step enlarged take their shapes' fat
 // boxes and mark their ancestors grown, then the partial rebuild and the new ranks.
-// gn: the tree's nodes in HBM; ranks: the world's per-shape rank array. Called by
-// all BLOCK lanes of the workgroup.
+// gn: the tree's nodes in HBM; ranks: the world's per-shape rank array; marked: the
+// enlarged leaves were taken care of before. Called by all BLOCK lanes of the workgroup.
 template <int BLOCK>
 __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape* shapes, int shapeCount,
-                                            int treeType, int* ranks, TreeWork w) {
+                                            int treeType, int* ranks, TreeWork w, bool marked) {
   const int lane = threadIdx.x;
   const int F = hd->fresh, P = hd->proxyCount, root = hd->root;
   if (P == 0 || root < 0 || root >= F) return;
@@ -240,8 +240,7 @@ __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape*
   __syncthreads();
   // enlarged leaves (b2DynamicTree_EnlargeProxy, S/dynamic_tree.c:827-866): a walk up
   // stops at a node another walk marked, whose ancestors that walk marks
-  bool any = false;
-  for (int k = lane; k < shapeCount; k += BLOCK) {
+  for (int k = lane; k < shapeCount && !marked; k += BLOCK) {
     Shape& sh = shapes[k];
     const int flags = sh.flags;
     if (!(flags & SF_TREE_PENDING) || sh.proxyKey < 0 || (sh.proxyKey & 3) != treeType) continue;
@@ -252,13 +251,11 @@ __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape*
       continue;
     }
     gn[leaf].box = sh.fat;
-    any = true;
     for (int p = w.links[leaf].z, g = 0; p >= 0 && p < F && g < F; p = w.links[p].z, ++g) {
       const int old = atomicOr(&w.links[p].w, TN_ENLARGED);
       if (old & TN_ENLARGED) break;
     }
   }
-  (void)any;
   __syncthreads();
   if (__syncthreads_or(bad) || hd->error) {
     if (lane == 0) hd->error = 2;

@@ -121,3 +121,18 @@ def test_frame_records(gpu, bodies, sleep, steps):
 def test_islands_sleep_and_split(gpu, bodies, steps):
     spec, geoms = container(bodies, 7 + bodies, sleep=True, speed=1.0)
     follow(spec, geoms, steps)
+
+
+# trees of more than 1,024 proxies are rebuilt beside the contacts and the solve: steps
+# queued one behind the other give what steps with a wait between them give
+@pytest.mark.parametrize("bodies,steps", [(1024, 8), (1025, 8), (2400, 8), (4200, 6)])
+def test_tree_rebuild_beside_the_solve(gpu, bodies, steps):
+    spec, geoms = container(bodies, 5 + bodies, bullets=0.02, speed=20.0)
+    follow(spec, geoms, 2)
+    queued, waited = F.Batch(spec), F.Batch(spec)
+    queued.step(steps=steps)
+    for _ in range(steps):
+        waited.step(steps=1)
+        assert waited.sync() == 0
+    assert queued.sync() == 0 and queued.error_bits() == 0
+    assert queued.export(0) == waited.export(0)
