@@ -885,7 +885,7 @@ static int treeLdsBytes(const HostWorld& hw, int limit) {
 }
 
 // lanes of the tree launch: about two proxies per lane per pass. From 1,024 proxies on the
-// work arrays leave LDS soon (1,400), and the passes wait for L2 instead: more lanes.
+// work arrays leave LDS soon (1,770), and the passes wait for L2 instead: more lanes.
 static int treeBlockFor(int proxies) {
   return proxies <= 96 ? 64 : (proxies <= 192 ? 128 : (proxies <= 1024 ? 256 : 1024));
 }

@@ -47,7 +47,7 @@ struct alignas(16) TreeHeader {
 };
 
 // ints of the device rebuild's work arrays for F node slots and P proxies
-F2D_HD long treeWorkInts(int F, int P) { return 4L * F + 20L * P + 160; }
+F2D_HD long treeWorkInts(int F, int P) { return 4L * (F > 2 * P ? F : 2 * P) + 14L * P + 160; }
 
 struct TreeRef {
   TreeHeader* h;

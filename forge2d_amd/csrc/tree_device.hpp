@@ -28,6 +28,14 @@
 // * Ranks. The query visits the items from the last to the first, each item's
 //   leaves in their old relative order: a leaf's new rank is the number of leaves
 //   of later items plus its old rank's offset within its item's interval.
+//
+// What bounds it: in LDS the workgroups that fit a compute unit (88 B a proxy: three of 500
+// proxies, as many as the registers allow, and trees of up to 1,770 proxies), and the chain
+// of dependent LDS accesses and barriers at each depth. The centre bounds of the ranges go
+// by register moves within rows of 16 lanes and one atomic a row; over 64 lanes with
+// shuffles that was 48 LDS instructions a pass. Both together: 160 worlds of 50 to 4,000
+// bodies 25.8 ms to 22.9 ms, 16,384 worlds 109.7 ms to 107.5 ms. In HBM the same passes
+// wait for L2 (2.6 ms for 20,000 proxies). Four waves per SIMD (128 registers) gained nothing.
 #pragma once
 
 #include "layout.hpp"
@@ -45,8 +53,10 @@ __device__ __forceinline__ float orderKeyFloat(int k) { return __int_as_float(k 
 
 // Work arrays of one tree rebuild for F node slots and P proxies (ints).
 struct TreeWork {
-  int4* links;     // [F] child1, child2, parent, flags | item place << 8
-  int* items;      // [P] build items, permuted by the partitions
+  int4* links;     // [F] child1, child2, parent, flags | item place << 8; until the build, whose
+                   //     ranges, left, right and itemHeight take their place
+  int* items;      // [P] build items by their first place, permuted by the partitions
+  int* nodeOf;     // [P] item nodes by first place
   float* cx;       // [P] item centres (cx, cy, seg and pre are contiguous: 16 B per item,
   float* cy;       //     reused as range boxes by the refit)
   int* seg;        // [P] range of each item place at the current depth, -1 when done
@@ -54,8 +64,8 @@ struct TreeWork {
   int* partner;    // [P] right-part places by rank; heights in the refit; final places in the ranks
   int4* ranges;    // [P] start, end, child1 links above, node id
   int* split;      // [P] split place
-  int* left;       // [P] child1 range index, or -1 - item node
-  int* right;      // [P] child2 range index, or -1 - item node
+  int* left;       // [P] child1 range index, or -1 - item
+  int* right;      // [P] child2 range index, or -1 - item
   int* bounds;     // [2P + 8] per range of a depth: centre bounds as order keys, then axis and
                    //     pivot (aliases byRank and lowOf, idle during the build)
   int* grown;      // [P] grown nodes in child1-first preorder
@@ -65,7 +75,7 @@ struct TreeWork {
   int* lowMark;    // [P] item place by the lower end of its rank interval
   int* levels;     // [P + 2] first range of each depth
   float4* itemBox; // [P] (aliases grown, byRank, lowOf, split) item boxes by first place, for the refit
-  int* itemHeight; // [P] item heights by first place
+  int* itemHeight; // [P] item heights by first place (in the links)
   int* counter;    // [4] range count
   int* sums;       // [16] per-wavefront partial sums of the block scans
 };
@@ -74,7 +84,11 @@ __device__ __forceinline__ TreeWork treeWorkAt(int* base, int F, int P) {
   TreeWork t;
   int* p = base;
   t.links = reinterpret_cast<int4*>(p);
-  p += 4L * F;
+  t.ranges = t.links;
+  t.left = p + 4L * P;
+  t.right = p + 5L * P;
+  t.itemHeight = p + 6L * P;
+  p += 4L * maxi(F, 2 * P);
   t.cx = reinterpret_cast<float*>(p);
   p += P;
   t.cy = reinterpret_cast<float*>(p);
@@ -83,15 +97,13 @@ __device__ __forceinline__ TreeWork treeWorkAt(int* base, int F, int P) {
   p += P;
   t.pre = p;
   p += P + 64;
-  t.ranges = reinterpret_cast<int4*>(p);
-  p += 4L * P;
   t.items = p;
+  p += P;
+  t.nodeOf = p;
   p += P;
   t.partner = p;
   p += P;
-  t.left = p;
-  p += P;
-  t.right = p;
+  t.leaves = p;
   p += P;
   t.grown = p;
   p += P;
@@ -104,10 +116,6 @@ __device__ __forceinline__ TreeWork treeWorkAt(int* base, int F, int P) {
   p += P;
   // item boxes for the refit, by first place, over grown..split (idle after the build)
   t.itemBox = reinterpret_cast<float4*>(t.grown);
-  t.itemHeight = p;
-  p += P;
-  t.leaves = p;
-  p += P;
   t.lowMark = p;
   p += P;
   t.levels = p;
@@ -136,24 +144,19 @@ __device__ __forceinline__ int waveInclusiveMax(int v, int lane) {
   return v;
 }
 
-// Minimum (or maximum) over the run of lanes that share `key` with this lane and
-// precede it: lanes of one key are consecutive (items of one range are consecutive
-// places), so the run's last lane holds the run's result.
-__device__ __forceinline__ int segMinUp(int v, int key, int lane) {
-  for (int d = 1; d < 64; d <<= 1) {
-    const int o = __shfl_up(v, d, 64);
-    const int k = __shfl_up(key, d, 64);
-    if (lane >= d && k == key) v = min(v, o);
-  }
-  return v;
+// v of the lane D places down in the lane's row of 16, or v itself in the row's first D
+// (a register move, not an LDS instruction like __shfl)
+template <int D>
+__device__ __forceinline__ int rowShift(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, 0x110 + D, 0xF, 0xF, false);
 }
-__device__ __forceinline__ int segMaxUp(int v, int key, int lane) {
-  for (int d = 1; d < 64; d <<= 1) {
-    const int o = __shfl_up(v, d, 64);
-    const int k = __shfl_up(key, d, 64);
-    if (lane >= d && k == key) v = max(v, o);
-  }
-  return v;
+// Minimum (or maximum) over the run of lanes of one range that precede this lane in its row:
+// items of one range are consecutive places, and `run` counts those before this lane in the
+// row. The run's last lane in each row holds that row's result.
+template <int D>
+__device__ __forceinline__ void rowMinMax(int4& v, int run) {
+  const int4 o = make_int4(rowShift<D>(v.x), rowShift<D>(v.y), rowShift<D>(v.z), rowShift<D>(v.w));
+  if (run >= D) v = make_int4(min(v.x, o.x), min(v.y, o.y), max(v.z, o.z), max(v.w, o.w));
 }
 
 // Block-wide scans over BLOCK lanes (BLOCK / 64 wavefronts): every lane of the
@@ -315,7 +318,8 @@ __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape*
       const int pos = count + prefix;
       const int node = w.byRank[r];
       const int lo = w.lowOf[r];
-      w.items[pos] = node;
+      w.items[pos] = pos;
+      w.nodeOf[pos] = node;
       w.leaves[pos] = r - lo + 1;
       w.lowMark[lo] = pos;
       w.links[node].w = (w.links[node].w & 0xFF) | (pos << 8);
@@ -353,7 +357,6 @@ __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape*
     }
   }
   if (lane == 0) {
-    w.ranges[0] = make_int4(0, count, 0, 0);
     w.levels[0] = 0;
     w.levels[1] = 1;
     w.counter[0] = 1;
@@ -369,7 +372,8 @@ __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape*
     if (lane == 0) hd->error = 2;
     return;
   }
-  if (lane == 0) w.ranges[0].w = w.grown[nGrown - 1];
+  // the links are not read any more
+  if (lane == 0) w.ranges[0] = make_int4(0, count, 0, w.grown[nGrown - 1]);
 
   // ---- the build, one depth at a time
   int begin = 0, end = 1, depth = 0, prevBegin = 0;
@@ -384,7 +388,7 @@ __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape*
     // bounds of every range of three or more items
     for (int base = 0; base < count; base += BLOCK) {
       const int i = base + lane;
-      int r = -1;
+      int r = -1, first = 0, last = 0;
       if (i < count) {
         r = w.seg[i];
         if (depth > 0) {
@@ -398,21 +402,25 @@ __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape*
         }
         if (r >= 0) {
           const int4 R = w.ranges[r];
-          if (R.y - R.x < 3) r = -1;
+          first = R.x;
+          last = R.y - 1;
+          if (last - first < 2) r = -1;
         }
       }
-      // one atomic per range and wavefront: reduce each run of lanes of one range first
-      const int wl = lane & 63;
+      // one atomic per range and row of 16 lanes
+      const int row = lane & 15, run = min(row, i - first);
       const int kx = r >= 0 ? floatOrderKey(w.cx[i]) : 0, ky = r >= 0 ? floatOrderKey(w.cy[i]) : 0;
-      const int mnx = segMinUp(kx, r, wl), mny = segMinUp(ky, r, wl);
-      const int mxx = segMaxUp(kx, r, wl), mxy = segMaxUp(ky, r, wl);
-      const int nextKey = __shfl_down(r, 1, 64);
-      if (r >= 0 && (wl == 63 || nextKey != r)) {
+      int4 m = make_int4(kx, ky, kx, ky);
+      rowMinMax<1>(m, run);
+      rowMinMax<2>(m, run);
+      rowMinMax<4>(m, run);
+      rowMinMax<8>(m, run);
+      if (r >= 0 && (row == 15 || i == last)) {
         int* bd = w.bounds + 4 * (r - begin);
-        atomicMin(bd + 0, mnx);
-        atomicMin(bd + 1, mny);
-        atomicMax(bd + 2, mxx);
-        atomicMax(bd + 3, mxy);
+        atomicMin(bd + 0, m.x);
+        atomicMin(bd + 1, m.y);
+        atomicMax(bd + 2, m.z);
+        atomicMax(bd + 3, m.w);
       }
     }
     __syncthreads();
@@ -501,8 +509,10 @@ __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape*
         made = (m - R.x >= 2 ? 1 : 0) + (R.y - m >= 2 ? 1 : 0);
       }
       // child ranges are numbered in range order (a block prefix of the children made)
-      int total;
-      const int slot = next + blockInclusiveAdd<BLOCK>(made, w.sums, &total) - made;
+      int total, both;
+      int slot = next + blockFlagPrefix<BLOCK>(made > 0, w.sums, &total);
+      slot += blockFlagPrefix<BLOCK>(made > 1, w.sums, &both);
+      total += both;
       next += total;
       if (k >= nl) continue;
       w.split[r] = m;
@@ -538,11 +548,9 @@ __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape*
 
   // ---- item boxes and heights, one read each, by first place
   for (int k = lane; k < count; k += BLOCK) {
-    const int node = w.items[k];
-    const int first = w.links[node].w >> 8;
-    const TreeNode& n = gn[node];
-    w.itemBox[first] = make_float4(n.box.lo.x, n.box.lo.y, n.box.hi.x, n.box.hi.y);
-    w.itemHeight[first] = n.height;
+    const TreeNode& n = gn[w.nodeOf[k]];
+    w.itemBox[k] = make_float4(n.box.lo.x, n.box.lo.y, n.box.hi.x, n.box.hi.y);
+    w.itemHeight[k] = n.height;
   }
   __syncthreads();
 
@@ -561,12 +569,12 @@ __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape*
           h[e] = w.partner[c[e]];
           id[e] = w.ranges[c[e]].w;
         } else {
-          id[e] = -1 - c[e];
-          if (id[e] < 0 || id[e] >= F) {
+          const int first = -1 - c[e];
+          if (first >= count) {
             valid = false;
             continue;
           }
-          const int first = w.links[id[e]].w >> 8;
+          id[e] = w.nodeOf[first];
           const float4 v = w.itemBox[first];
           b[e] = AABB{{v.x, v.y}, {v.z, v.w}};
           h[e] = w.itemHeight[first];
@@ -606,7 +614,7 @@ __device__ __forceinline__ void rebuildTree(TreeHeader* hd, TreeNode* gn, Shape*
   // each item's leaves in their old order. partner: final place of each first place;
   // left: leaves at each final place; right: leaves at later final places
   for (int k = lane; k < count; k += BLOCK) {
-    const int first = w.links[w.items[k]].w >> 8;
+    const int first = w.items[k];
     w.partner[first] = k;
     w.left[k] = w.leaves[first];
   }
