@@ -841,7 +841,7 @@ static void freeDevice(Batch& b) {
 
 // Dynamic LDS bytes a step launch may ask for on the current device: the device's
 // LDS per workgroup (160 KiB on gfx950, 64 KiB when the query fails) less 4 KiB
-// for the step kernels' own static LDS (at most 1.3 KiB), since a dispatch whose
+// for the step kernels' own static LDS (at most 3.3 KiB), since a dispatch whose
 // static plus dynamic LDS exceeds the device limit is refused.
 static int deviceLdsLimit() {
   static int limit = 0;
@@ -2741,9 +2741,9 @@ int f2dg_autotune(void* h, float dt, int subSteps, int steps, float* msOut) {
     for (int s = 0; s < (5 - nCands) * steps; ++s) {
       if (f2d_launch_step(&b->dev.view, &sp, c.dList, c.count, b->stream, &c.launch) != 0) return -1;
     }
-    // LDS room for constraint lanes: more keeps more worlds' constraints on chip,
-    // less lets more workgroups share a compute unit; every class runs the same
-    // number of trial steps, so all worlds advance equally
+    // LDS sizes of the solve launch: less lets more workgroups share a compute unit (no stage
+    // uses more than the first); every class runs the same number of trial steps, so all
+    // worlds advance equally
     const float lanesPerBody[4] = {0.0f, 0.5f, 1.0f, 2.0f};
     best = 1e30f;
     int bestLds = c.launch.solveLds;

@@ -4,16 +4,19 @@
 //
 //   pairs     sort-and-sweep over fat AABBs (LDS bitonic sort of lower-x keys),
 //             new pairs emitted with wavefront atomics, ordered like the
-//             reference's move buffer, then contacts created serially
+//             reference's move buffer, then contacts created a lane each and linked
+//             into the bodies' lists in pair order
 //             (S/broad_phase.c:160-474, S/contact.c:186-328)
-//   collide   one contact per lane: overlap test, manifold, warm-start id
+//   collide   one contact per lane, gathered by manifold kind: overlap test,
+//             manifold, warm-start id
 //             matching (S/world.c:357-445, S/contact.c:472-633)
 //   state     contact begin/end/destroy in ascending contact id with persistent
 //             greedy colouring (S/world.c:587-690, S/constraint_graph.c:68-212)
 //   solve     prepare, then substeps x (integrate velocities, warm start, solve,
 //             integrate positions, relax), restitution, store; overflow colour
 //             first in each stage, then one colour per barrier, one constraint
-//             per lane, body states resident in LDS (S/solver.c:929-1106)
+//             per lane and colour, contacts in registers and body states in LDS
+//             where the world fits (S/solver.c:929-1106)
 //   finalize  one body per lane: transforms, AABBs, fat-AABB enlarge and the
 //             next move buffer (S/solver.c:543-726, 1819-1911)
 //
@@ -1779,8 +1782,12 @@ __device__ __forceinline__ void listJoints(const WorldPtrs& w, SharedState& sh, 
   }
 }
 
-// Contact lanes a lane of the resident solve keeps in registers: three (84 VGPRs of the
-// 128 that leave four wavefronts a SIMD), so a workgroup holds three contacts a lane.
+// Contact lanes a lane of the resident solve keeps in registers, so a workgroup holds three
+// contacts a lane: three wavefronts a SIMD have 168 VGPRs each. 4,096 pyramids (24 steps) and
+// 2,048 piles (32 steps) took 83.8 and 37.3 ms with the constraints in LDS or HBM, 36.7 and
+// 20.7 ms so. At four wavefronts: two a lane 38.5 and 19.1 ms (64 worlds 8 % slower, too),
+// three 45.7 and 25.2 ms (69 spills). At two, five or six a lane with half the lanes: 37.5
+// and 19.7 ms at best, and latency suffers.
 constexpr int kResidentLanes = 3;
 
 // The solver stages of a world whose contacts fit the workgroup's registers
@@ -2310,8 +2317,10 @@ __device__ void stepContext(const WorldHeader* h, const StepParams& sp, SolveCtx
 // LDS hold the sort-and-sweep arrays (28 B per shape) with the existing-pair hash
 // set behind them, then the new-pair sort (12 B per pair); larger worlds use their
 // global scratch region and walk the contact lists instead.
-// Four waves per SIMD: the compiler keeps the manifold code within 128 VGPRs
-// (measured faster than the 148-VGPR, three-wave build on the 16k-world workload).
+// What bounds it is the latency of scattered record reads, at three wavefronts a SIMD (155
+// VGPRs; the manifold code spills 80 at four, which cost what the occupancy gained). Contacts
+// gathered by manifold kind and long sweeps a wavefront each: 2,048 piles 20.4 ms to 18.0 ms,
+// 160 worlds of 50 to 4,000 bodies 50.6 ms to 44.3 ms, 4,096 pyramids 37.6 ms to 33.8 ms.
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void collideKernel(BatchView b, StepParams sp, const int* worldList, int ldsBytes) {
   __shared__ SharedState sh;
@@ -3291,7 +3300,8 @@ __global__ __launch_bounds__(kQueryLanes) void explodeKernel(BatchView b, const 
 // What a frame of one world reads back, written to pinned host memory behind the step:
 // the error bits, and the moved bodies in the finalize's order (their body events). A
 // frame then needs one wait and no copies: it took two waits and nineteen copies, 4 us
-// each on the device and as much again on the host.
+// each on the device and as much again on the host: ten bodies 342 us a frame to 85 us, 820
+// bodies 568 us to 234 us.
 __global__ __launch_bounds__(256) void frameKernel(BatchView b, int world, int bodyCap, int* head,
                                                    FrameRecord* records) {
   const WorldHeader* h = b.worlds + world;

@@ -506,7 +506,8 @@ const char* f2dg_last_error(void* batch);
 /* autotuner: per size class, times `steps` steps with 64, 128 and 256 lanes per world (and
  * 512 and 1024 for classes of more than 256 shapes) and keeps the fastest (ms_out[3]
  * optional: whole-batch ms per 64/128/256 candidate), then times 4 solve
- * LDS sizes (room for 0, 0.5, 1 and 2 constraint lanes per body) and keeps the fastest;
+ * LDS sizes (the body terms, and 0.5, 1 and 2 constraint lanes per body more, which no
+ * stage uses since contacts stay in registers or HBM) and keeps the fastest;
  * classes with 3 lane candidates run 2 x steps untimed steps more, so every world advances by
  * 9 x steps trial steps; returns the largest class's lanes */
 int f2dg_autotune(void* batch, float dt, int sub_steps, int steps, float* ms_out);
@@ -526,8 +527,8 @@ int f2dg_set_block(void* batch, int block);
 int f2dg_get_block(void* batch);
 /* force the workgroup size of size class `cls` (index into f2dg_size_classes) */
 int f2dg_set_class_block(void* batch, int cls, int block);
-/* force the solve launch's dynamic LDS bytes of size class `cls` (body terms of its
- * largest world + constraint lanes; worlds whose lanes do not fit keep them in HBM) */
+/* force the solve launch's dynamic LDS bytes of size class `cls` (body terms and
+ * joints of its largest world; worlds that do not fit keep less of them in LDS) */
 int f2dg_set_class_solve_lds(void* batch, int cls, int bytes);
 /* aggregate counts after f2dg_sync (10 longs): [awake bodies, shapes, touching contacts,
  * touching points, restitution contacts, restitution points, joints, overflow contacts,
