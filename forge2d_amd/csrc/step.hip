@@ -1288,8 +1288,10 @@ constexpr int kChangeChunk = 32;
 // the records that its gathering touched to be near when the lane comes to them.
 // A pile of 20,000 bodies 94.1 ms to 89.6 ms for 16 steps, 160 worlds of 50 to 4,000 bodies
 // 35.3 ms to 30.4 ms for 24.
-// serialW: a workgroup-shared copy of w for the out-of-line island calls, so the world
-// pointers stay in registers elsewhere instead of a per-lane stack copy.
+// serialW: a workgroup-shared copy of the world pointers for the out-of-line island calls,
+// so they stay in registers elsewhere instead of a per-lane stack copy. Its colours are the
+// LDS copy too: writing that copy back and reading it again around every woken set cost as
+// much as the world is large (8,000 sets of 16,000 bodies woken in one step: 4.4 s, and 74 ms so).
 template <int BLOCK>
 __device__ void statePhase(const WorldPtrs& w, SharedState& sh, WorldPtrs& serialW, char* lds, int ldsBytes) {
   const int n = sh.changedCount;
@@ -1305,16 +1307,11 @@ __device__ void statePhase(const WorldPtrs& w, SharedState& sh, WorldPtrs& seria
     c0.colorCounts = colors;
     c0.colorBits = reinterpret_cast<uint32_t*>(colors + kColorListHeader);
   }
-  auto loadColors = [&](int first, int step) {
-    for (int k = first; k < kOverflowIndex; k += step) colors[k] = w.colorCounts[k];
-    for (int k = first; k < colorWords; k += step) colors[kColorListHeader + k] = (int)w.colorBits[k];
-  };
-  auto storeColors = [&](int first, int step) {
-    for (int k = first; k < kOverflowIndex; k += step) w.colorCounts[k] = colors[k];
-    for (int k = first; k < colorWords; k += step) w.colorBits[k] = (uint32_t)colors[kColorListHeader + k];
-  };
-  if (n > 0 && cached) loadColors(threadIdx.x, BLOCK);
-  if (threadIdx.x == 0) serialW = w;
+  if (n > 0 && cached) {
+    for (int k = threadIdx.x; k < kOverflowIndex; k += BLOCK) colors[k] = w.colorCounts[k];
+    for (int k = threadIdx.x; k < colorWords; k += BLOCK) colors[kColorListHeader + k] = (int)w.colorBits[k];
+  }
+  if (threadIdx.x == 0) serialW = c0;
   int nBegin = 0, nEnd = 0;  // thread 0's
   for (int base = 0; base < n; base += cap) {
     const int m = min(cap, n - base);
@@ -1377,9 +1374,7 @@ __device__ void statePhase(const WorldPtrs& w, SharedState& sh, WorldPtrs& seria
             setB = w.sims[r.bodyB].setIndex;
           }
           if ((setA == kAwakeSet && setB >= kFirstSleepingSet) || (setB == kAwakeSet && setA >= kFirstSleepingSet)) {
-            if (cached) storeColors(0, 1);
             linkContact(serialW, id);
-            if (cached) loadColors(0, 1);
             woke = true;
           } else {
             linkRootedIslands(w.isl, id, r.islandA, r.islandB, (r.bits & CR_ONE_ISLAND) != 0);
@@ -1404,7 +1399,10 @@ __device__ void statePhase(const WorldPtrs& w, SharedState& sh, WorldPtrs& seria
     }
     __syncthreads();
   }
-  if (n > 0 && cached) storeColors(threadIdx.x, BLOCK);
+  if (n > 0 && cached) {
+    for (int k = threadIdx.x; k < kOverflowIndex; k += BLOCK) w.colorCounts[k] = colors[k];
+    for (int k = threadIdx.x; k < colorWords; k += BLOCK) w.colorBits[k] = (uint32_t)colors[kColorListHeader + k];
+  }
   if (threadIdx.x == 0) {
     h->beginCount = nBegin;
     h->endCount = nEnd;

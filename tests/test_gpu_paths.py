@@ -6,6 +6,7 @@ compares it, bit for bit, with the oracle stepping the device's previous state.
 """
 import ctypes
 import os
+import time
 
 import numpy as np
 import pytest
@@ -23,9 +24,10 @@ GEOM_BYTES = 148
 
 
 def container(bodies: int, seed: int, bullets: float = 0.0, sleep: bool = False, speed: float = 0.0,
-              columns: int = 0) -> tuple[bytes, bytes]:
+              columns: int = 0, asleep: int = 0) -> tuple[bytes, bytes]:
     """(spec, geometry records) of a world of `bodies` dynamic bodies in rows in a
-    container, their shapes drawn from the "mixed" fixture's dynamic ones."""
+    container, their shapes drawn from the "mixed" fixture's dynamic ones; the first
+    `asleep` are created asleep."""
     src, _, _ = load_fixture("mixed")
     (_, fb, fs, _), = scenes.parse(src)
     fg = np.load(os.path.join(GOLDEN, "mixed.npz"))["geoms"].reshape(-1, GEOM_BYTES)
@@ -46,6 +48,7 @@ def container(bodies: int, seed: int, bullets: float = 0.0, sleep: bool = False,
     b["flags"][1:] |= np.where(rng.random(bodies) < bullets, scenes.BF_BULLET, 0).astype(np.int32)
     s = np.concatenate([fs[walls], fs[pick]])
     s["body"][:len(walls)], s["body"][len(walls):] = 0, 1 + at
+    b["flags"][1:1 + asleep] &= ~scenes.BF_AWAKE
     h = scenes.world_header(sleep=sleep)
     h["body_count"], h["shape_count"] = len(b), len(s)
     spec = scenes.MAGIC + np.array([1, 0], "<i4").tobytes() + h.tobytes() + b.tobytes() + s.tobytes()
@@ -121,6 +124,39 @@ def test_frame_records(gpu, bodies, sleep, steps):
 def test_islands_sleep_and_split(gpu, bodies, steps):
     spec, geoms = container(bodies, 7 + bodies, sleep=True, speed=1.0)
     follow(spec, geoms, steps)
+
+
+# every sleeping body is a set of its own, and a body falls on each: hundreds of sets wake in
+# one state loop, among contacts that begin without one
+@pytest.mark.parametrize("sets,steps", [(30, 30), (400, 16)])
+def test_sets_woken_together(gpu, sets, steps):
+    spec, geoms = container(2 * sets, 61 + sets, sleep=True, speed=2.0, columns=sets, asleep=sets)
+    follow(spec, geoms, steps)
+
+
+# four times the sleeping boxes, each woken in the first step, take about four times as long
+# (16 times if a wake cost what the world is large); the larger world of the two is the one
+# whose loop the cost would rule
+def test_waking_a_set_costs_the_set(gpu):
+    def first_step(sets: int) -> float:
+        w = scenes.World(scenes.world_header(sleep=True))
+        for i in range(sets):
+            w.add_box(w.add_body(scenes.DYNAMIC, 2.0 * i, 0.5, flags=scenes.BF_ENABLE_SLEEP), 0.5, 0.5)
+        for i in range(sets):
+            w.add_box(w.add_body(scenes.DYNAMIC, 2.0 * i, 1.51), 0.5, 0.5)
+        b = F.Batch([w])
+        b.upload()
+        b.synchronize()
+        t = time.perf_counter()
+        b.step(steps=1)
+        b.synchronize()
+        t = time.perf_counter() - t
+        assert b.sync() == 0 and b.counters(0)["touching"] == sets
+        return t
+
+    first_step(10)  # the library's code objects are loaded
+    small, large = first_step(500), first_step(2000)
+    assert large < 8 * small, (small, large)
 
 
 # trees of more than 1,024 proxies are rebuilt beside the contacts and the solve: steps
