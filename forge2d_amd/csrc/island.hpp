@@ -128,7 +128,7 @@ F2D_HD void addJointToIsland(IslandCtx& c, int islandId, int jid) {
 
 // Union-find root with path halving: every island left on the way up points to
 // its grandparent (the walk of S/island.c:150-196 and :547-566)
-F2D_HD int islandRoot(IslandCtx& c, int id) {
+F2D_HD int islandRoot(const IslandCtx& c, int id) {
   Island* is = &c.islands[id];
   // parents form a forest; the walk is bounded by the island count all the same
   for (int guard = c.h->islandCount; is->parent != -1 && guard > 0; --guard) {

@@ -159,6 +159,30 @@ def test_waking_a_set_costs_the_set(gpu):
     assert large < 8 * small, (small, large)
 
 
+# a plank made last touches every box in one step, and each contact links the islands so far
+# below the next box's: four times the boxes take about four times as long (16 times if each
+# link walked the links before it)
+def test_links_of_one_island_with_many(gpu):
+    def state_loop(boxes: int) -> float:
+        w = scenes.World(scenes.world_header())
+        for i in range(boxes):
+            w.add_box(w.add_body(scenes.DYNAMIC, 1.2 * i, 0.5), 0.5, 0.5)
+        w.add_box(w.add_body(scenes.DYNAMIC, 0.6 * boxes, 1.25), 0.6 * boxes + 1.0, 0.25)
+        b = F.Batch([w])
+        b.upload()
+        b.synchronize()
+        t = time.perf_counter()
+        b.step(steps=1, phases=F.PH_PAIRS | F.PH_COLLIDE | F.PH_STATE)
+        b.synchronize()
+        t = time.perf_counter() - t
+        assert b.sync() == 0 and b.counters(0)["touching"] == boxes
+        return t
+
+    state_loop(10)  # the library's code objects are loaded
+    small, large = state_loop(4000), state_loop(16000)
+    assert large < 8 * small, (small, large)
+
+
 # trees of more than 1,024 proxies are rebuilt beside the contacts and the solve: steps
 # queued one behind the other give what steps with a wait between them give
 @pytest.mark.parametrize("bodies,steps", [(1024, 8), (1025, 8), (2400, 8), (4200, 6)])
