@@ -2771,14 +2771,14 @@ int f2dg_autotune(void* h, float dt, int subSteps, int steps, float* msOut) {
   return b->classes.empty() ? b->launch.block : b->classes.back().launch.block;
 }
 
-// Force the solve launch's dynamic LDS bytes of one size class (at least its body
-// terms; at most the device's LDS per workgroup).
+// Force the solve launch's dynamic LDS bytes of one size class: 0, or from the body states
+// of its largest world (every size that the automatic choice takes) to the device's LDS per
+// workgroup.
 int f2dg_set_class_solve_lds(void* h, int cls, int bytes) {
   Batch* b = static_cast<Batch*>(h);
   if (!b || cls < 0 || cls >= (int)b->classes.size() || bytes < 0 || bytes > deviceLdsLimit()) return -1;
   SizeClass& c = b->classes[cls];
-  const int bodies = std::max(c.maxBodies, 1) * (int)(sizeof(BodyState) + sizeof(BodyConst));
-  if (bytes < bodies && bytes != 0) return -1;
+  if (bytes != 0 && bytes < std::max(c.maxBodies, 1) * (int)sizeof(BodyState)) return -1;
   c.launch.solveLds = bytes;
   return 0;
 }

@@ -527,8 +527,11 @@ int f2dg_set_block(void* batch, int block);
 int f2dg_get_block(void* batch);
 /* force the workgroup size of size class `cls` (index into f2dg_size_classes) */
 int f2dg_set_class_block(void* batch, int cls, int block);
-/* force the solve launch's dynamic LDS bytes of size class `cls` (body terms and
- * joints of its largest world; worlds that do not fit keep less of them in LDS) */
+/* force the solve launch's dynamic LDS bytes of size class `cls`: 0, or from 32 bytes a body
+ * of its largest world to the device's LDS per workgroup (any solve LDS bytes that
+ * f2dg_size_classes reports are accepted). A world's contacts stay in registers where its
+ * 64 * (bodies + 1) bytes and its joints with their lists (292 bytes each) fit; with 32 bytes
+ * a body its states lie in LDS; with less, nothing does */
 int f2dg_set_class_solve_lds(void* batch, int cls, int bytes);
 /* aggregate counts after f2dg_sync (10 longs): [awake bodies, shapes, touching contacts,
  * touching points, restitution contacts, restitution points, joints, overflow contacts,

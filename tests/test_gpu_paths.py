@@ -92,6 +92,26 @@ def test_solver_stages(gpu, bodies, block, steps):
     follow(spec, geoms, steps, b)
 
 
+# the reported solve LDS of every class can be given back, as can what the sizes between the
+# solver's forms are; less than the body states cannot
+def test_solve_lds_given_back(gpu):
+    specs = [container(n, 3 + n)[0] for n in (40, 200, 500, 900, 1100, 3000, 6000)]
+    b = F.Batch(scenes.MAGIC + np.array([len(specs), 0], "<i4").tobytes() + b"".join(s[16:] for s in specs))
+    b.upload()
+    classes = b.size_classes()
+    assert len(classes) == 7
+    for k, c in enumerate(classes):
+        for size in (c["solve_lds"], 0, 32 * c["max_bodies"], 64 * (c["max_bodies"] + 1)):
+            if size <= 159744:
+                b.set_class_solve_lds(k, size)
+                assert b.size_classes()[k]["solve_lds"] == size
+        for size in (32 * c["max_bodies"] - 1, 163841, -1):
+            with pytest.raises(RuntimeError):
+                b.set_class_solve_lds(k, size)
+        b.set_class_solve_lds(k, c["solve_lds"])
+    assert b.size_classes() == classes
+
+
 # a frame's body events come from records written behind the step, or, once the mirror was
 # read back, from the mirror: the same, for worlds around the record kernel's 256 lanes
 @pytest.mark.parametrize("bodies,sleep,steps", [(1, True, 90), (255, False, 4), (256, True, 4), (700, False, 4)])
