@@ -2173,13 +2173,15 @@ long f2dg_device_bytes(void* h) {
   return b ? (long)b->dev.bytes : -1;
 }
 
-// Step every world of the batch `steps` times: one launch per step, one workgroup per world.
-// Lane candidates of a size class for online tuning: 64, 128 and 256 lanes per
-// world, 256, 512 and 1024 for worlds of more than 512 shapes or bodies.
-static int laneCandidate(const SizeClass& c, int k) {
-  static const int small[3] = {64, 128, 256}, large[3] = {256, 512, 1024};
-  return c.limit > 512 ? large[k] : small[k];
-}
+// Lane candidates of a size class for online tuning, the size it starts with among them:
+// 64, 128 and 256 lanes per world, 128, 256 and 512 for worlds of more than 256 shapes or
+// bodies, 256, 512 and 1024 for more than 512. The solve keeps three contacts a lane in
+// registers, so a size left out is lost to a class that needs it: without 512 lanes, 1,024
+// worlds of 406 stacked boxes went from 0.81 ms a step to 1.04 ms with their first round.
+// 64 lanes are no loss there: 2,000 worlds of 257 to 509 bodies, 49 / 603 / 650 touching
+// contacts each, take 1.38 / 2.94 / 2.43 ms at 64, 1.16 / 2.14 / 1.96 at 128, 1.07 / 1.52 /
+// 1.47 at 256 and 1.47 / 1.97 / 1.66 at 512.
+static int laneCandidate(const SizeClass& c, int k) { return (c.limit > 512 ? 256 : (c.limit > 256 ? 128 : 64)) << k; }
 
 // One online tuning round: three steps, step k with every class at its k-th lane
 // candidate, the classes one after another on the batch's stream with HIP events
@@ -2215,6 +2217,7 @@ static int tuneRound(Batch& b, const StepParams& sp) {
   return 0;
 }
 
+// Step every world of the batch `steps` times: one launch per step, one workgroup per world.
 int f2dg_step(void* h, float dt, int subSteps, int steps, int phases) {
   Batch* b = static_cast<Batch*>(h);
   if (!b) return -1;

@@ -512,8 +512,8 @@ const char* f2dg_last_error(void* batch);
  * 9 x steps trial steps; returns the largest class's lanes */
 int f2dg_autotune(void* batch, float dt, int sub_steps, int steps, float* ms_out);
 /* online lane tuning of f2dg_step: every `period` steps (0: off), a round of three ordinary
- * steps runs each size class at 64, 128 and 256 lanes per world (256, 512 and 1024 for
- * classes of more than 512 shapes), the classes one after another, timed with HIP events,
+ * steps runs each size class at 64, 128 and 256 lanes per world (128, 256 and 512 for classes
+ * of more than 256 shapes, 256, 512 and 1024 for more than 512), the classes one after another, timed with HIP events,
  * and each class keeps its fastest; as worlds settle and gather contacts the best size
  * changes, and the lanes never change results */
 int f2dg_set_online_tuning(void* batch, int period);
