@@ -857,23 +857,26 @@ static int deviceLdsLimit() {
   return limit;
 }
 
-// Lay out all worlds in flat arrays and allocate the device batch.
-// Dynamic LDS of a solve launch, for the class's largest world. Up to 1,024 bodies: the
-// body states and per-step body terms (64 B a body and one slot for the static bodies)
-// and the joints with their colour lists, which lets a world's contacts stay in the
-// workgroup's registers (solveResident). Larger worlds have more contacts than that and
-// keep only the body states (32 B a body) in LDS, up to the limit. lanesPerBody: room
-// beyond that, which no stage uses (0; the autotuner's trial sizes).
-static int solveLdsBytes(int maxBodies, int maxJoints, float lanesPerBody, int limit) {
+// Dynamic LDS of a solve launch, for the class's largest world, in one of two sizes. full: the
+// body states and per-step body terms (64 B a body and one slot for the static bodies) and the
+// joints with their colour lists, which lets a world's contacts stay in the workgroup's
+// registers where there are at most three a lane (solveResident). Else the body states alone
+// (32 B a body), the contacts streamed; a size over the limit falls to the next, 0 last.
+static int solveLdsBytes(int maxBodies, int maxJoints, bool full, int limit) {
   const long bodies = std::max(maxBodies, 1);
-  const long states = bodies * (long)sizeof(BodyState);
   long total = (bodies + 1) * (long)(sizeof(BodyState) + sizeof(BodyConst)) +
                (long)maxJoints * (long)(sizeof(Joint) + sizeof(int));
-  if (bodies > 1024 || total > limit) total = states;
+  if (!full || total > limit) total = bodies * (long)sizeof(BodyState);
   if (total > limit) return 0;
-  total += (long)(lanesPerBody * (float)bodies) * 4L * CN_FIELD_COUNT;
   return (int)std::min<long>((total + 255) & ~255L, limit);
 }
+
+// Classes of up to this many bodies take the full size by themselves. Above it the workgroup
+// has 1,024 lanes all the same, whose registers hold the contacts no better than L2 does, and
+// a settled world soon has more than three a lane: 64 worlds of 1,100 bodies (2,162 contacts)
+// solve in 0.223 ms a step with the full size and in 0.208 ms with the states, of 1,400 bodies
+// (2,761 contacts) in 0.246 and 0.250 ms; 1,900 bodies stream either way (3,797 contacts).
+constexpr int kFullSolveBodies = 1024;
 
 // LDS for the tree kernel's work arrays of a world's larger moving tree (worlds that
 // need more than `limit` work from HBM)
@@ -896,6 +899,7 @@ static int treeBlockFor(int proxies) {
 // step for 370, 160 worlds of 50 to 4,000 bodies 40.6 ms for 32.4, for the queues shared).
 constexpr int kTreeBesideProxies = 1024;
 
+// Lay out all worlds in flat arrays and allocate the device batch.
 static int commit(Batch& b) {
   freeDevice(b);
   long nb = 0, ns = 0, nc = 0, nj = 0, ncol = 0, nscratch = 0, nisl = 0, ntree = 0, nclist = 0;
@@ -1027,7 +1031,7 @@ static int commit(Batch& b) {
   b.launch.treeBlock = treeBlockFor(maxProxies);
   int maxJoints = 0;
   for (const HostWorld& hw : b.worlds) maxJoints = std::max(maxJoints, (int)hw.joints.size());
-  b.launch.solveLds = solveLdsBytes(maxBodies, maxJoints, 0.0f, deviceLdsLimit());
+  b.launch.solveLds = solveLdsBytes(maxBodies, maxJoints, maxBodies <= kFullSolveBodies, deviceLdsLimit());
   if (b.launch.block == 0) b.launch.block = maxShapes <= 640 ? 64 : 256;
   // Full-batch launches dispatch the largest worlds first (longest-processing-time
   // order), so the last wave of workgroups holds the smallest worlds and the
@@ -1079,7 +1083,7 @@ static int commit(Batch& b) {
       c.launch.continuousChunks = c.maxBodies > 1024 ? (c.maxBodies + 63) / 64 : 0;
       // worlds of many thousand bodies run their solve stages over many workgroups
       c.launch.wideChunks = c.maxBodies > 4096 ? (c.maxBodies + 255) / 256 : 0;
-      c.launch.solveLds = solveLdsBytes(c.maxBodies, c.maxJoints, 0.0f, deviceLdsLimit());
+      c.launch.solveLds = solveLdsBytes(c.maxBodies, c.maxJoints, c.maxBodies <= kFullSolveBodies, deviceLdsLimit());
       c.launch.treeLds = 0;
       int maxProxies = 0;
       for (int i : members[k]) {
@@ -2703,7 +2707,7 @@ int f2dg_world_counters(void* h, int world, int* out) {
 
 // Workgroup-size autotuner: for each size class, time `steps` steps of that
 // class's worlds with each candidate size (64, 128, 256 lanes per world) and keep
-// the fastest. msOut (optional, 3 floats) receives the whole-batch ms per
+// the fastest, then with each solve LDS size. msOut (optional, 3 floats) receives the whole-batch ms per
 // candidate summed over classes. The trial steps advance every world by the same
 // number of steps; results do not depend on the workgroup size.
 int f2dg_autotune(void* h, float dt, int subSteps, int steps, float* msOut) {
@@ -2744,15 +2748,15 @@ int f2dg_autotune(void* h, float dt, int subSteps, int steps, float* msOut) {
     for (int s = 0; s < (5 - nCands) * steps; ++s) {
       if (f2d_launch_step(&b->dev.view, &sp, c.dList, c.count, b->stream, &c.launch) != 0) return -1;
     }
-    // LDS sizes of the solve launch: less lets more workgroups share a compute unit (no stage
-    // uses more than the first); every class runs the same number of trial steps, so all
-    // worlds advance equally
-    const float lanesPerBody[4] = {0.0f, 0.5f, 1.0f, 2.0f};
-    best = 1e30f;
-    int bestLds = c.launch.solveLds;
+    // the two LDS sizes of the solve launch, in turn: the other one replaces the class's own
+    // only if it was faster both times, so that no choice is made by noise. Every class runs
+    // the same number of trial steps, so all worlds advance equally
+    const int own = c.launch.solveLds, full = solveLdsBytes(c.maxBodies, c.maxJoints, true, deviceLdsLimit());
+    const int other = own != full ? full : solveLdsBytes(c.maxBodies, c.maxJoints, false, deviceLdsLimit());
+    float slowestOther = 0.0f, fastestOwn = 1e30f;
     for (int k = 0; k < 4; ++k) {
       LaunchConfig cfg = c.launch;
-      cfg.solveLds = solveLdsBytes(c.maxBodies, c.maxJoints, lanesPerBody[k], deviceLdsLimit());
+      cfg.solveLds = (k & 1) ? other : own;
       F2D_HIP(hipEventRecord(e0, b->stream));
       for (int s = 0; s < steps; ++s) {
         if (f2d_launch_step(&b->dev.view, &sp, c.dList, c.count, b->stream, &cfg) != 0) return -1;
@@ -2761,11 +2765,10 @@ int f2dg_autotune(void* h, float dt, int subSteps, int steps, float* msOut) {
       F2D_HIP(hipEventSynchronize(e1));
       float ms = 0.0f;
       F2D_HIP(hipEventElapsedTime(&ms, e0, e1));
-      if (ms < best) {
-        best = ms;
-        bestLds = cfg.solveLds;
-      }
+      if (k & 1) slowestOther = std::max(slowestOther, ms);
+      else fastestOwn = std::min(fastestOwn, ms);
     }
+    const int bestLds = slowestOther < fastestOwn ? other : own;
     c.launch.solveLds = bestLds;
   }
   (void)hipEventDestroy(e0);

@@ -505,11 +505,11 @@ int f2dg_import_world(void* batch, int world, const void* snapshot, long bytes);
 const char* f2dg_last_error(void* batch);
 /* autotuner: per size class, times `steps` steps with 64, 128 and 256 lanes per world (and
  * 512 and 1024 for classes of more than 256 shapes) and keeps the fastest (ms_out[3]
- * optional: whole-batch ms per 64/128/256 candidate), then times 4 solve
- * LDS sizes (the body terms, and 0.5, 1 and 2 constraint lanes per body more, which no
- * stage uses since contacts stay in registers or HBM) and keeps the fastest;
- * classes with 3 lane candidates run 2 x steps untimed steps more, so every world advances by
- * 9 x steps trial steps; returns the largest class's lanes */
+ * optional: whole-batch ms per 64/128/256 candidate), then times the two solve LDS sizes (the
+ * body terms and joints, or the body states alone) twice each in turn and changes the class's
+ * own only if the other was faster both times; classes with 3 lane candidates run 2 x steps
+ * untimed steps more, so every world advances by 9 x steps trial steps; returns the largest
+ * class's lanes */
 int f2dg_autotune(void* batch, float dt, int sub_steps, int steps, float* ms_out);
 /* online lane tuning of f2dg_step: every `period` steps (0: off), a round of three ordinary
  * steps runs each size class at 64, 128 and 256 lanes per world (128, 256 and 512 for classes

@@ -72,6 +72,22 @@ def test_autotune_advances_every_world_equally(gpu):
     assert steps == {18}, steps
 
 
+def test_autotune_keeps_to_the_solver_s_lds_sizes(gpu):
+    """The solve LDS size that the autotuner leaves is one of the two that the solver tells
+    apart: body terms (64 bytes a body and for one slot more) and joints (292 bytes each),
+    or 32 bytes a body."""
+    worlds = [scenes.container_world(n, 20.0, 40.0, 7100 + n, chains=c)
+              for n, c in ((30, 0), (100, 1), (220, 2), (450, 0), (800, 3), (1300, 2))]
+    b = F.Batch(worlds)
+    b.upload()
+    b.autotune(steps=1)
+    assert b.sync() == 0
+    for c, w in zip(b.size_classes(), worlds):
+        n = len(w.bodies)
+        sizes = (32 * n, 64 * (n + 1) + 292 * len(w.joints))
+        assert c["max_bodies"] == n and c["solve_lds"] in [(k + 255) // 256 * 256 for k in sizes], c
+
+
 def test_online_tuning_does_not_change_results(gpu):
     """Online lane tuning (trial rounds every 5 steps, classes stepped one after
     another at each candidate size) gives the same bits as plain stepping."""
