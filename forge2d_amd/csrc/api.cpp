@@ -981,7 +981,7 @@ static int commit(Batch& b) {
       devAlloc(d, &v.contacts, nc) || devAlloc(d, &v.freeIds, nc) || devAlloc(d, &v.overflow, nc) ||
       devAlloc(d, &v.pairs, nc) || devAlloc(d, &v.pairShapes, nc) || devAlloc(d, &v.joints, nj) ||
       devAlloc(d, &v.colorBits, ncol) || devAlloc(d, &v.cons, (size_t)nc * CN_FIELD_COUNT) ||
-      devAlloc(d, &v.scratch, nscratch) || devAlloc(d, &v.ccolor, nc) || devAlloc(d, &v.staticShapes, ns) || devAlloc(d, &v.sweepOrder, ns) ||
+      devAlloc(d, &v.scratch, nscratch) || devAlloc(d, &v.staticShapes, ns) || devAlloc(d, &v.sweepOrder, ns) ||
       devAlloc(d, &v.events, 3 * nc) || devAlloc(d, &v.islandData, std::max(nisl, 4L)) ||
       devAlloc(d, &v.contactLinks, nc) || devAlloc(d, &v.treeHdrs, 3L * W) ||
       devAlloc(d, &v.colorLists, std::max(nclist, 1L)) ||
@@ -1148,7 +1148,6 @@ static int upload(Batch& b) {
   std::vector<WorldHeader> headers(b.worlds.size());
   long totalContacts = 0;
   for (const HostWorld& hw : b.worlds) totalContacts = std::max<long>(totalContacts, hw.hdr.contactOffset + hw.hdr.contactCap);
-  std::vector<int8_t> ccolor(totalContacts, -1);
   long totalShapes = 0;
   for (const HostWorld& hw : b.worlds) totalShapes = std::max<long>(totalShapes, hw.hdr.shapeOffset + hw.hdr.shapeCount);
   std::vector<int> staticShapes(std::max<long>(totalShapes, 1), 0);
@@ -1192,11 +1191,7 @@ static int upload(Batch& b) {
     F2D_HIP(hipMemcpyAsync(v.treeRanks + h.shapeOffset, hw.treeRanks.data(), sizeof(int) * h.shapeCount, hipMemcpyHostToDevice, s));
     F2D_HIP(hipMemcpyAsync(v.geoms + h.shapeOffset, hw.geoms.data(), sizeof(ShapeGeom) * h.shapeCount, hipMemcpyHostToDevice, s));
     F2D_HIP(hipMemcpyAsync(v.contacts + h.contactOffset, hw.contacts.data(), sizeof(Contact) * h.contactCap, hipMemcpyHostToDevice, s));
-    for (int k = 0; k < h.contactCap; ++k) {
-      const Contact& c = hw.contacts[k];
-      ccolor[h.contactOffset + k] = (int8_t)(c.shapeA >= 0 ? c.color : -1);
-      if (k < (int)hw.links.size()) links[h.contactOffset + k] = hw.links[k];
-    }
+    std::copy_n(hw.links.begin(), std::min<size_t>(hw.links.size(), h.contactCap), links.begin() + h.contactOffset);
     {
       IslandRegion r = islandRegion(h.islandCap, h.bodyCount);
       int* base = islandData.data() + h.islandOffset;
@@ -1233,7 +1228,6 @@ static int upload(Batch& b) {
   F2D_HIP(hipMemcpyAsync(v.treeNodes, treeNodes.data(), sizeof(TreeNode) * treeNodes.size(), hipMemcpyHostToDevice, b.stream));
   F2D_HIP(hipMemcpyAsync(v.treeFreed, treeFreed.data(), sizeof(int) * treeFreed.size(), hipMemcpyHostToDevice, b.stream));
   F2D_HIP(hipMemcpyAsync(v.worlds, headers.data(), sizeof(WorldHeader) * headers.size(), hipMemcpyHostToDevice, b.stream));
-  F2D_HIP(hipMemcpyAsync(v.ccolor, ccolor.data(), ccolor.size(), hipMemcpyHostToDevice, b.stream));
   F2D_HIP(hipMemcpyAsync(v.staticShapes, staticShapes.data(), sizeof(int) * totalShapes, hipMemcpyHostToDevice, b.stream));
   F2D_HIP(hipMemcpyAsync(v.sweepOrder, sweepOrder.data(), sizeof(int) * totalShapes, hipMemcpyHostToDevice, b.stream));
   F2D_HIP(hipMemcpyAsync(v.islandData, islandData.data(), sizeof(int) * islandData.size(), hipMemcpyHostToDevice, b.stream));

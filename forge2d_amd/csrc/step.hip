@@ -45,7 +45,6 @@ constexpr int kWideTableInts = 64;
 struct SharedState {
   int colorCount[kGraphColorCount];
   int colorStart[kGraphColorCount + 1];
-  int colorFill[kGraphColorCount];
   int jointColorCount[kGraphColorCount];
   int jointColorStart[kGraphColorCount + 1];
   int jointColorFill[kGraphColorCount];
@@ -196,7 +195,6 @@ struct WorldPtrs {
   Cons cons;
   int* scratch;
   float4* sapBoxes;
-  int8_t* ccolor;
   int* events;
   int4* links;      // contact island links and solver set
   int* sweepOrder;
@@ -223,7 +221,6 @@ __device__ WorldPtrs worldPtrs(const BatchView& b, WorldHeader* h) {
   w.cons.f = b.cons + 4L * h->constraintOffset;
   w.cons.stride = b.consStride;
   w.scratch = b.scratch + h->scratchOffset;
-  w.ccolor = b.ccolor + h->contactOffset;
   w.events = b.events + 3L * h->contactOffset;
   w.sapBoxes = b.sapBoxes + h->shapeOffset;
   w.sweepOrder = b.sweepOrder + h->shapeOffset;
@@ -347,12 +344,11 @@ __device__ void considerPair(const WorldPtrs& w, int* pairCount, int s, int t, c
 // creation order), with the result of a serial loop over them: ids are the LIFO
 // pool's pops in creation order (free list top first, then fresh ids), so each pair's
 // id follows from its rank among the pairs that get a contact; the records are filled
-// in parallel. pk is reused for the oriented shapes and pv for the ids. edges: LDS for
-// edgeCap edges of the body contact lists (it may lie over pk).
+// in parallel. pv is reused for the ids. edges: LDS for edgeCap edges of the body contact
+// lists (it may lie over the pairs' sort keys).
 constexpr int kLinkedPairs = 1024;
 template <int BLOCK>
-__device__ void createContacts(const WorldPtrs& w, SharedState& sh, uint64_t* pk, int* pv, int count, int4* edges,
-                               int edgeCap) {
+__device__ void createContacts(const WorldPtrs& w, SharedState& sh, int* pv, int count, int4* edges, int edgeCap) {
   WorldHeader* h = w.hdr;
   const int freeCount = h->freeCount, fresh = h->contactCount, cap = h->contactCap;
   int created = 0;
@@ -393,7 +389,6 @@ __device__ void createContacts(const WorldPtrs& w, SharedState& sh, uint64_t* pk
         }
       }
       const int kind = valid ? manifoldKind(w.geoms[a].type, w.geoms[bsh].type) : 0;
-      pk[i] = ((uint64_t)(uint32_t)a << 32) | (uint32_t)bsh;
       pv[i] = id;
       if (id >= 0) {
         const Shape& A = w.shapes[a];
@@ -405,7 +400,6 @@ __device__ void createContacts(const WorldPtrs& w, SharedState& sh, uint64_t* pk
         c.simFlags = ((A.flags | B.flags) & SF_PRESOLVE) ? SIM_PRESOLVE : 0;
         c.color = -1;
         c.localIndex = -1;
-        w.ccolor[id] = -1;
         c.bodyA = A.body;
         c.bodyB = B.body;
         zeroManifold(c.m);
@@ -568,8 +562,7 @@ __device__ void sweepShapes(const WorldPtrs& w, LongSweeps& sh, const float4* bo
 // launch (sweepKernel) spreads the sweep over many workgroups, and mode 2 creates the
 // pairs it found, in the same order.
 template <int BLOCK>
-__device__ void pairsPhase(const WorldPtrs& w, SharedState& sh, char* lds, int ldsShapes, int ldsPairs, int ldsBytes,
-                           int mode) {
+__device__ void pairsPhase(const WorldPtrs& w, SharedState& sh, char* lds, int ldsPairs, int ldsBytes, int mode) {
   WorldHeader* h = w.hdr;
   const int n = h->shapeCount;
   if (threadIdx.x == 0) sh.pairCount = 0;
@@ -592,7 +585,6 @@ __device__ void pairsPhase(const WorldPtrs& w, SharedState& sh, char* lds, int l
   // and the existing-pair hash set when they fit
   const int np = nextPow2(max(n, 4));
   const bool inLds = 28L * np <= (long)ldsBytes;
-  (void)ldsShapes;
   uint64_t* keys = inLds ? reinterpret_cast<uint64_t*>(lds) : reinterpret_cast<uint64_t*>(w.scratch);
   // keys (lower fat x, shape id) laid out in the last step's sweep order, which is
   // nearly sorted when bodies move little per step
@@ -710,7 +702,7 @@ __device__ void pairsPhase(const WorldPtrs& w, SharedState& sh, char* lds, int l
     }
     __syncthreads();
     bitonicSort<BLOCK>(pk, pv, pp);
-    createContacts<BLOCK>(w, sh, pk, pv, count, reinterpret_cast<int4*>(lds),
+    createContacts<BLOCK>(w, sh, pv, count, reinterpret_cast<int4*>(lds),
                           (pairsInLds ? 8 * ldsPairs : ldsBytes) / (int)sizeof(int4));
   }
   __syncthreads();
@@ -952,7 +944,6 @@ __device__ void addContactToGraphBodies(const WorldPtrs& w, int id, int bodyA, i
     }
   }
   c.color = color;
-  w.ccolor[id] = (int8_t)color;
   if (color == kOverflowIndex) {
     WorldHeader* h = w.hdr;
     if (h->overflowCount >= h->contactCap) {
@@ -1005,7 +996,6 @@ __device__ void removeContactFromGraph(const WorldPtrs& w, int id) {
   }
   c.color = -1;
   c.localIndex = -1;
-  w.ccolor[id] = -1;
 }
 
 // b2DestroyContact, S/contact.c:337-454 (no island or event bookkeeping on the device)
@@ -2343,16 +2333,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void
     h->moveBodyCount = 0;  // body move events start empty each step (S/world.c:709)
   }
   __syncthreads();
-  int ldsShapes = 1;
-  while (ldsShapes * 2 * 28 <= ldsBytes) ldsShapes *= 2;
-  if (ldsShapes * 28 > ldsBytes) ldsShapes = 0;
   int ldsPairs = 1;
   while (ldsPairs * 2 * 12 <= ldsBytes) ldsPairs *= 2;
   if (ldsPairs * 12 > ldsBytes) ldsPairs = 0;
   if (sp.phases & PH_PAIRS) {
-    pairsPhase<BLOCK>(w, sh, lds, ldsShapes, ldsPairs, ldsBytes, (sp.phases & PH_PAIRS_PREP) ? 1 : 0);
+    pairsPhase<BLOCK>(w, sh, lds, ldsPairs, ldsBytes, (sp.phases & PH_PAIRS_PREP) ? 1 : 0);
   } else if (sp.phases & PH_PAIRS_FINISH) {
-    pairsPhase<BLOCK>(w, sh, lds, ldsShapes, ldsPairs, ldsBytes, 2);
+    pairsPhase<BLOCK>(w, sh, lds, ldsPairs, ldsBytes, 2);
   }
   if (sp.phases & PH_COLLIDE) collidePhase<BLOCK>(w, sh, bins, lds, ldsBytes, (sp.phases & PH_CONTACTS_DONE) != 0);
   if (sp.phases & PH_STATE) statePhase<BLOCK>(w, sh, serialW, lds, ldsBytes);
@@ -3493,8 +3480,7 @@ static int launchBlock(const BatchView* b, const StepParams* sp, const int* worl
     if (sp->phases & PH_FINALIZE) {
       StepParams f = *sp;
       f.phases = sp->phases & ~PH_SOLVE;
-      hipLaunchKernelGGL(solveKernel<BLOCK>, dim3(nWorlds), dim3(BLOCK), cfg->solveLds, stream, *b, f, worldList,
-                         cfg->solveLds);
+      hipLaunchKernelGGL(solveKernel<BLOCK>, dim3(nWorlds), dim3(BLOCK), 0, stream, *b, f, worldList, 0);
     }
   } else if (sp->phases & (PH_SOLVE | PH_FINALIZE)) {
     hipLaunchKernelGGL(solveKernel<BLOCK>, dim3(nWorlds), dim3(BLOCK), cfg->solveLds, stream, *b, *sp, worldList,
