@@ -30,9 +30,8 @@ pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HARNESS = os.path.join(ROOT, "oracle", "_ref", "ref_harness")
 
-# (scene, steps): the last two exceed the 64 KB of LDS a world may use, so their
-# body states (pyramid48) and their sort-and-sweep too (container2600) run from
-# global memory
+# pyramid48 and container2600 keep only their body states in LDS, and container2600 (whose
+# shapes are too many for the sort in LDS) sorts and sweeps in global memory
 SCENES = {
     "pyramid25": lambda: scenes.pyramid_world(25),
     "pyramid48": lambda: scenes.pyramid_world(48),

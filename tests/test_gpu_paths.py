@@ -24,10 +24,11 @@ GEOM_BYTES = 148
 
 
 def container(bodies: int, seed: int, bullets: float = 0.0, sleep: bool = False, speed: float = 0.0,
-              columns: int = 0, asleep: int = 0) -> tuple[bytes, bytes]:
+              columns: int = 0, asleep: int = 0, shapeless: int = 0) -> tuple[bytes, bytes]:
     """(spec, geometry records) of a world of `bodies` dynamic bodies in rows in a
     container, their shapes drawn from the "mixed" fixture's dynamic ones; the first
-    `asleep` are created asleep."""
+    `asleep` are created asleep, and `shapeless` bodies without shapes follow them. One
+    static body, the container's, comes before."""
     src, _, _ = load_fixture("mixed")
     (_, fb, fs, _), = scenes.parse(src)
     fg = np.load(os.path.join(GOLDEN, "mixed.npz"))["geoms"].reshape(-1, GEOM_BYTES)
@@ -49,6 +50,10 @@ def container(bodies: int, seed: int, bullets: float = 0.0, sleep: bool = False,
     s = np.concatenate([fs[walls], fs[pick]])
     s["body"][:len(walls)], s["body"][len(walls):] = 0, 1 + at
     b["flags"][1:1 + asleep] &= ~scenes.BF_AWAKE
+    extra = np.zeros(shapeless, scenes.BODY_DT)
+    extra["qc"], extra["flags"], extra["type"] = 1.0, scenes.BF_ENABLE_SLEEP | scenes.BF_AWAKE, scenes.DYNAMIC
+    extra["px"], extra["vx"], extra["w"], extra["lin_damp"] = np.arange(shapeless), 0.5, 1.0, 0.25
+    b = np.concatenate([b, extra])
     h = scenes.world_header(sleep=sleep)
     h["body_count"], h["shape_count"] = len(b), len(s)
     spec = scenes.MAGIC + np.array([1, 0], "<i4").tobytes() + h.tobytes() + b.tobytes() + s.tobytes()
@@ -79,17 +84,45 @@ def test_bullets(gpu, bodies, bullets, sleep, steps):
 
 
 # the solver stages: contacts in registers (up to three a lane), or streamed with the bodies
-# in LDS (more contacts than that, or worlds above 1,024 bodies) or with nothing in LDS;
-# lanes a power of two from 64, worlds on both sides of what they hold
+# in LDS (more contacts than that, or worlds above 1,024 bodies, as 1,024 here are with their
+# container), or a launch a stage (above 4,096 bodies: 4,095 are the most that is not); lanes
+# a power of two from 64, worlds on both sides of what they hold
 @pytest.mark.parametrize("bodies,block,steps", [(1, 64, 30), (2, 1024, 30), (63, 64, 40), (64, 64, 40), (130, 64, 60),
                                                 (130, 128, 60), (500, 64, 40), (500, 256, 40), (500, 512, 40),
                                                 (1000, 1024, 30), (1023, 512, 20), (1024, 1024, 20), (3000, 1024, 12),
-                                                (4096, 256, 6), (4097, 1024, 6)])
+                                                (4095, 1024, 6), (4096, 256, 6), (4097, 1024, 6)])
 def test_solver_stages(gpu, bodies, block, steps):
     spec, geoms = container(bodies, 23 + bodies, speed=4.0)
     b = F.Batch(spec)
     b.set_block(block)
     follow(spec, geoms, steps, b)
+
+
+# the solver stages streamed with nothing in LDS, as in worlds whose states do not fit: the size
+# set to 0, or so many more bodies than shapes that the scratch region has no room for the
+# per-step body terms. Stepped one by one, a batch's worlds take the size of its largest
+@pytest.mark.parametrize("bodies,shapeless,solve_lds,block,steps", [
+    (1, 0, 0, 64, 30), (130, 0, 0, 64, 60), (500, 0, 0, 512, 30), (1500, 0, 0, 1024, 12), (40, 1100, None, 256, 40),
+    (300, 3000, None, 1024, 20)])
+def test_solver_stages_without_lds(gpu, bodies, shapeless, solve_lds, block, steps):
+    spec, geoms = container(bodies, 29 + bodies, speed=4.0, shapeless=shapeless)
+    b = F.Batch(spec)
+    b.upload()
+    b.set_block(block)
+    if solve_lds is not None:
+        b.set_class_solve_lds(0, solve_lds)
+    follow(spec, geoms, steps, b)
+
+
+def test_worlds_stepped_one_by_one_without_lds(gpu):
+    specs = [container(n, 31 + n, speed=4.0)[0] for n in (200, 1500, 5000)]  # 160 KB of states in the last
+    spec = scenes.MAGIC + np.array([len(specs), 0], "<i4").tobytes() + b"".join(s[16:] for s in specs)
+    one, all_ = F.Batch(spec), F.Batch(spec)
+    one.step_each(steps=8)
+    all_.step(steps=8)
+    assert one.sync() == 0 and all_.sync() == 0
+    for w in range(len(specs)):
+        assert one.export(w) == all_.export(w), w
 
 
 # the reported solve LDS of every class can be given back, as can what the sizes between the
