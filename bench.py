@@ -78,6 +78,25 @@ def algorithmic_bytes(st: dict) -> dict:
             "step": float(solve + collide + tree)}
 
 
+def roofline(launch_ms: dict, nbytes: dict, workload: str) -> dict:
+    """The longest kernel against the HBM peak, by the bytes that its counters read in the
+    workload's committed counter runs (profiles/pmc_<workload>.json, over its steps
+    traffic_steps); null without them. algorithmic_gbs is the rate of the stage
+    model's bytes, which the kernel does not move: bodies stay in LDS and contacts in
+    registers between the stages. The step is latency-bound, well below either."""
+    dominant = max(launch_ms, key=launch_ms.get)
+    pmc = load_pmc(workload)
+    traffic = pmc.get(dominant, {}).get("hbm_bytes_per_launch") if pmc else None
+    ms = launch_ms[dominant]
+    achieved = traffic / (ms * 1e-3) / 1e9 if traffic else None
+    model = nbytes.get(dominant)
+    return {"bound": "latency", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": achieved / HBM_PEAK_GBS if achieved else None, "traffic": traffic,
+            "traffic_steps": pmc.get("window") if traffic else None, "kernel": dominant,
+            "launch_ms": ms, "algorithmic_bytes_per_launch": model,
+            "algorithmic_gbs": model / (ms * 1e-3) / 1e9 if model else None}
+
+
 def load_pmc(workload: str):
     path = os.path.join(ROOT, "profiles", f"pmc_{workload}.json")
     if os.path.exists(path):
@@ -279,6 +298,8 @@ def main():
                (f" --solve-lds {args.solve_lds}" if args.solve_lds else ""))
         res = pmc_summary(args.pmc_summary[0], args.pmc_summary[1], EV_STEPS, args.trace_dispatches,
                           args.workload, cmd, mib)
+        first = args.warmup + 9 * 4 + args.steps + LATENCY_STEPS  # as kernel_profile steps them
+        res["window"] = [first, first + EV_STEPS - 1]
         with open(os.path.join(ROOT, "profiles", f"pmc_{args.workload}.json"), "w") as f:
             json.dump(res, f, indent=1)
         print(json.dumps(res, indent=1))
@@ -404,13 +425,11 @@ def main():
         raise RuntimeError("device reported a capacity error")
     st_ev = batch.stats()
     nbytes = algorithmic_bytes(st_ev)
-    dominant = max(launch_ms, key=launch_ms.get)
-    achieved = nbytes[dominant] / (launch_ms[dominant] * 1e-3) / 1e9
+    roof = roofline(launch_ms, nbytes, args.workload)
+    dominant = roof["kernel"]
     step_gbs = nbytes["step"] / (sum(launch_ms.values()) * 1e-3) / 1e9
-    pmc = load_pmc(args.workload)
-    traffic = pmc.get(dominant, {}).get("hbm_bytes_per_launch") if pmc else None
     log(f"[bench] kernel ms per step (steps {ev_first}..{ev_first + EV_STEPS - 1}) {launch_ms}, "
-        f"algorithmic bytes {nbytes}, {dominant} {achieved:.0f} GB/s")
+        f"algorithmic bytes {nbytes}, {dominant} {roof['achieved']} GB/s by counters")
 
     cpu = None
     if not args.no_cpu:
@@ -455,9 +474,7 @@ def main():
         "batched_vs_per_world": (value / per_world["value"]) if per_world else None,
         "batched_vs_cpu": (value / cpu["value"]) if cpu else None,
         "batched_vs_cpu_one_thread": (value / cpu["t1"]["value"]) if cpu else None,
-        "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "kernel": dominant,
-                     "launch_ms": launch_ms[dominant], "algorithmic_bytes_per_launch": nbytes[dominant],
+        "roofline": {**roof,
                      "window": {"steps": [ev_first, ev_first + EV_STEPS - 1],
                                 "dispatches_per_step": len(batch.size_classes()),
                                 "contacts_per_body": st_ev["contacts"] / max(awake, 1),
@@ -465,7 +482,7 @@ def main():
                                          "in a kernel trace of this command"},
                      "other_kernel": {k: {"launch_ms": launch_ms[k], "algorithmic_bytes_per_launch": nbytes.get(k)}
                                       for k in launch_ms if k != dominant},
-                     "step_achieved_gbs": step_gbs},
+                     "step_algorithmic_gbs": step_gbs},
         "cpu_baseline": cpu,
         "queries": queries,
     }
@@ -489,23 +506,17 @@ def kernel_profile(args, batch, awake, desc):
         raise RuntimeError("device reported a capacity error")
     st = batch.stats()
     nbytes = algorithmic_bytes(st)
-    dominant = max(launch_ms, key=launch_ms.get)
-    achieved = nbytes[dominant] / (launch_ms[dominant] * 1e-3) / 1e9
+    roof = roofline(launch_ms, nbytes, args.workload)
     classes = batch.size_classes()
-    pmc = load_pmc(args.workload)
     out = {
         "metric": METRIC, "mode": "kernel-profile", "n_gpus": 1, "steps": EV_STEPS, "warmup": pre,
         "dtype": "f32", "config": {"workload": f"{args.workload}: {desc}", "awake_bodies": awake,
                                    "size_classes": classes, "stats": st},
         "kernel_ms_per_step": launch_ms,
         "dispatches_per_kernel": {k: len(classes) * EV_STEPS for k in launch_ms},
-        "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": pmc.get(dominant, {}).get("hbm_bytes_per_launch") if pmc else None,
-                     "kernel": dominant, "launch_ms": launch_ms[dominant],
-                     "algorithmic_bytes_per_launch": nbytes[dominant], "window": [pre, pre + EV_STEPS - 1]},
+        "roofline": {**roof, "window": [pre, pre + EV_STEPS - 1]},
     }
-    log(f"[bench] kernel profile: {launch_ms} ms per step, {dominant} {achieved:.0f} GB/s")
+    log(f"[bench] kernel profile: {launch_ms} ms per step, {roof['kernel']} {roof['achieved']} GB/s by counters")
     print(json.dumps(out), flush=True)
 
 
