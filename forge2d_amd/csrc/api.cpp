@@ -888,7 +888,9 @@ static int treeLdsBytes(const HostWorld& hw, int limit) {
 }
 
 // lanes of the tree launch: about two proxies per lane per pass. From 1,024 proxies on the
-// work arrays leave LDS soon (1,770), and the passes wait for L2 instead: more lanes.
+// work arrays leave LDS soon (1,770), and the passes wait for L2 instead: more lanes (1,100 /
+// 1,700 / 2,000 / 20,000 proxies: 0.106 / 0.127 / 0.33 / 2.99 ms, with 256 lanes 0.147 / 0.214
+// / 0.51 / 6.13 ms).
 static int treeBlockFor(int proxies) {
   return proxies <= 96 ? 64 : (proxies <= 192 ? 128 : (proxies <= 1024 ? 256 : 1024));
 }

@@ -1777,11 +1777,17 @@ __device__ __forceinline__ void listJoints(const WorldPtrs& w, SharedState& sh, 
 }
 
 // Contact lanes a lane of the resident solve keeps in registers, so a workgroup holds three
-// contacts a lane: three wavefronts a SIMD have 168 VGPRs each. 4,096 pyramids (24 steps) and
-// 2,048 piles (32 steps) took 83.8 and 37.3 ms with the constraints in LDS or HBM, 36.7 and
-// 20.7 ms so. At four wavefronts: two a lane 38.5 and 19.1 ms (64 worlds 8 % slower, too),
-// three 45.7 and 25.2 ms (69 spills). At two, five or six a lane with half the lanes: 37.5
-// and 19.7 ms at best, and latency suffers.
+// contacts a lane: up to 512 lanes, three wavefronts a SIMD have 168 VGPRs each (11 spilled).
+// 4,096 pyramids (24 steps) and 2,048 piles (32 steps) took 83.8 and 37.3 ms with the
+// constraints in LDS or HBM, 36.7 and 20.7 ms so. At four wavefronts: two a lane 38.5 and
+// 19.1 ms (64 worlds 8 % slower, too), three 45.7 and 25.2 ms (69 spills). At two, five or six
+// a lane with half the lanes: 37.5 and 19.7 ms at best, and latency suffers.
+// A workgroup of 1,024 lanes is four wavefronts a SIMD whatever is asked for, and its 128
+// VGPRs with 69 spilled do not hold three contacts. Classes above 512 run it all the same: one
+// world of 600 / 820 / 900 bodies (1,195 / 2,380 / 1,808 contacts) solves in 148 / 153 / 177 us
+// a step so, streamed at 1,024 lanes in 130 / 146 / 184 us, at 512 lanes in 104 / 147 / 186 us
+// (the first of them resident, the others too many contacts for that); 1,024 pyramids of 820
+// boxes at once take 2.34 to 2.46 ms a step, streamed 1.97 to 2.30 ms.
 constexpr int kResidentLanes = 3;
 
 // The solver stages of a world whose contacts fit the workgroup's registers
@@ -2192,7 +2198,10 @@ __device__ __forceinline__ void finalizeBodies(const WorldPtrs& w, SharedState& 
 // the joints: then the contacts stay in registers (solveResident) unless there are too
 // many, or overflow constraints, or joints of other types (out-of-line calls). Otherwise
 // the states alone (32 B a body), otherwise nothing; contacts and joints then stream from
-// L2 (solveStreamed).
+// L2 (solveStreamed). One distance joint takes a pyramid of 78 / 300 / 666 boxes from 87 / 106
+// / 195 us a step to 122 / 151 / 201 us that way; 256 worlds of 102 / 302 / 502 bodies with 10
+// / 50 / 90 overflow contacts each take 0.24 / 0.63 / 1.03 ms. With the constraints in LDS, as
+// far as they fitted, that was 215 / 375 / 431 us and 0.41 / 1.36 / 2.30 ms.
 template <int BLOCK>
 __device__ __forceinline__ void solveAndFinalize(const WorldPtrs& w, SharedState& sh, char* lds, const SolveCtx& ctx,
                                                  int phases, int ldsBytes) {
@@ -2311,8 +2320,9 @@ __device__ void stepContext(const WorldHeader* h, const StepParams& sp, SolveCtx
 // LDS hold the sort-and-sweep arrays (28 B per shape) with the existing-pair hash
 // set behind them, then the new-pair sort (12 B per pair); larger worlds use their
 // global scratch region and walk the contact lists instead.
-// What bounds it is the latency of scattered record reads, at three wavefronts a SIMD (155
-// VGPRs; the manifold code spills 80 at four, which cost what the occupancy gained). Contacts
+// What bounds it is the latency of scattered record reads, at three wavefronts a SIMD (154
+// VGPRs; the manifold code spills 80 at four, which cost what the occupancy gained; the 1,024
+// lanes of classes above 512 are four in any case, with 48 spilled). Contacts
 // gathered by manifold kind and long sweeps a wavefront each: 2,048 piles 20.4 ms to 18.0 ms,
 // 160 worlds of 50 to 4,000 bodies 50.6 ms to 44.3 ms, 4,096 pyramids 37.6 ms to 33.8 ms.
 template <int BLOCK>

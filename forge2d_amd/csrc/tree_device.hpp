@@ -34,8 +34,10 @@
 // of dependent LDS accesses and barriers at each depth. The centre bounds of the ranges go
 // by register moves within rows of 16 lanes and one atomic a row; over 64 lanes with
 // shuffles that was 48 LDS instructions a pass. Both together: 160 worlds of 50 to 4,000
-// bodies 25.8 ms to 22.9 ms, 16,384 worlds 109.7 ms to 107.5 ms. In HBM the same passes
-// wait for L2 (2.6 ms for 20,000 proxies). Four waves per SIMD (128 registers) gained nothing.
+// bodies 25.8 ms to 22.9 ms (24 steps, both on one state), 16,384 worlds 109.7 ms to 107.5 ms.
+// In HBM the same passes wait for L2 (3.0 ms for 20,000 proxies). Up to 256 lanes four waves
+// per SIMD (128 registers) gained nothing over three; 1,024 lanes are four in any case, with
+// 90 registers spilled, and still rebuild large trees in half the time of 256.
 #pragma once
 
 #include "layout.hpp"
