@@ -78,27 +78,32 @@ def algorithmic_bytes(st: dict) -> dict:
             "step": float(solve + collide + tree)}
 
 
-def roofline(launch_ms: dict, nbytes: dict, workload: str) -> dict:
-    """The longest kernel against the HBM peak, by the bytes that its counters read in the
-    workload's committed counter runs (profiles/pmc_<workload>.json, over its steps
-    traffic_steps); null without them. algorithmic_gbs is the rate of the stage
-    model's bytes, which the kernel does not move: bodies stay in LDS and contacts in
-    registers between the stages. The step is latency-bound, well below either."""
+def roofline(launch_ms: dict, nbytes: dict, workload: str, first: int) -> dict:
+    """The longest kernel against the HBM peak, by the bytes that its counters read over the
+    same steps in the committed counter runs (profiles/pmc_<workload>_step<first>.json); null
+    where no run covers them. algorithmic_gbs is the rate of the stage model's bytes, which
+    the kernel does not move: bodies stay in LDS and contacts in registers between the
+    stages. The step is latency-bound, well below either."""
     dominant = max(launch_ms, key=launch_ms.get)
-    pmc = load_pmc(workload)
+    pmc = load_pmc(workload, first)
     traffic = pmc.get(dominant, {}).get("hbm_bytes_per_launch") if pmc else None
     ms = launch_ms[dominant]
     achieved = traffic / (ms * 1e-3) / 1e9 if traffic else None
     model = nbytes.get(dominant)
     return {"bound": "latency", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS if achieved else None, "traffic": traffic,
-            "traffic_steps": pmc.get("window") if traffic else None, "kernel": dominant,
+            "kernel": dominant,
             "launch_ms": ms, "algorithmic_bytes_per_launch": model,
             "algorithmic_gbs": model / (ms * 1e-3) / 1e9 if model else None}
 
 
-def load_pmc(workload: str):
-    path = os.path.join(ROOT, "profiles", f"pmc_{workload}.json")
+def pmc_path(workload: str, first: int) -> str:
+    return os.path.join(ROOT, "profiles", f"pmc_{workload}_step{first}.json")
+
+
+def load_pmc(workload: str, first: int):
+    """The workload's committed counter runs over the steps from `first` on, or None."""
+    path = pmc_path(workload, first)
     if os.path.exists(path):
         with open(path) as f:
             return json.load(f)
@@ -289,18 +294,19 @@ def main():
     ap.add_argument("--trace-dispatches", type=int, default=5, metavar="N",
                     help="dispatches per step kernel per step in the traced run (its size-class count)")
     ap.add_argument("--pmc-summary", nargs=2, default=None, metavar=("FETCH_CSV", "WRITE_CSV"),
-                    help="write profiles/pmc_<workload>.json from two counter runs of --kernel-profile and exit")
+                    help="write profiles/pmc_<workload>_step<first>.json from two counter runs of --kernel-profile "
+                         "(with their --warmup and --steps) and exit")
     args = ap.parse_args()
     if args.pmc_summary:
         mib = args.copy_calibration or 512
         cmd = (f"rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE -- python3 -u bench.py --kernel-profile --workload "
-               f"{args.workload} --copy-calibration {mib}" + (f" --lanes {args.lanes}" if args.lanes else "") +
+               f"{args.workload} --warmup {args.warmup} --steps {args.steps} --copy-calibration {mib}" + (f" --lanes {args.lanes}" if args.lanes else "") +
                (f" --solve-lds {args.solve_lds}" if args.solve_lds else ""))
         res = pmc_summary(args.pmc_summary[0], args.pmc_summary[1], EV_STEPS, args.trace_dispatches,
                           args.workload, cmd, mib)
         first = args.warmup + 9 * 4 + args.steps + LATENCY_STEPS  # as kernel_profile steps them
         res["window"] = [first, first + EV_STEPS - 1]
-        with open(os.path.join(ROOT, "profiles", f"pmc_{args.workload}.json"), "w") as f:
+        with open(pmc_path(args.workload, first), "w") as f:
             json.dump(res, f, indent=1)
         print(json.dumps(res, indent=1))
         return
@@ -425,7 +431,7 @@ def main():
         raise RuntimeError("device reported a capacity error")
     st_ev = batch.stats()
     nbytes = algorithmic_bytes(st_ev)
-    roof = roofline(launch_ms, nbytes, args.workload)
+    roof = roofline(launch_ms, nbytes, args.workload, ev_first)
     dominant = roof["kernel"]
     step_gbs = nbytes["step"] / (sum(launch_ms.values()) * 1e-3) / 1e9
     log(f"[bench] kernel ms per step (steps {ev_first}..{ev_first + EV_STEPS - 1}) {launch_ms}, "
@@ -506,7 +512,7 @@ def kernel_profile(args, batch, awake, desc):
         raise RuntimeError("device reported a capacity error")
     st = batch.stats()
     nbytes = algorithmic_bytes(st)
-    roof = roofline(launch_ms, nbytes, args.workload)
+    roof = roofline(launch_ms, nbytes, args.workload, pre)
     classes = batch.size_classes()
     out = {
         "metric": METRIC, "mode": "kernel-profile", "n_gpus": 1, "steps": EV_STEPS, "warmup": pre,
